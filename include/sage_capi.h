@@ -104,8 +104,8 @@ int sage_quant_kv(const void* k, int64_t ksb, int64_t kss, int64_t ksh, const vo
 
 /*
  * Work plan of sage_attn_fwd on the current device: query tiles (128 rows of one batch and head, numbered
- * ((b * H + h) * ceil(Sq / 128) + tile)) below *n_full run whole; each later tile splits its key tiles of 64 keys into
- * *chunks contiguous ranges merged by a second kernel.  *workspace_bytes is the workspace the split needs (0 when
+ * ((b * H + h) * ceil(Sq / 128) + tile)) below *n_full run whole; each later tile splits the key tiles of 64 keys into
+ * *chunks contiguous ranges merged by a second kernel (causal launches split every tile or none).  *workspace_bytes is the workspace the split needs (0 when
  * nothing is split).  Output pointers may be NULL.  No counterpart in the reference (its launch is one workgroup per
  * query tile, src/rdna4_sage/_attention.py:133-139).
  */
@@ -212,7 +212,8 @@ int sage_forward_masked(const void* q, int64_t qsb, int64_t qss, int64_t qsh, co
  * the process ends); the caller passes only the inputs and the output, with sage_forward's meaning.  For callers
  * that cannot call hipMalloc or an allocating library (code under HIP graph capture, tight serving loops, harnesses
  * that forbid it).  No counterpart in the reference.  A shape whose intermediates and workspace exceed the array
- * returns SAGE_ERR_INVALID (128 MiB holds e.g. [1, 24, 4608, 128], 69 MB, and [2, 32/8, 8192, 128], 103 MB).  Every
+ * returns SAGE_ERR_INVALID, where the split tiles' partial state is left out (every tile whole) if only it does not
+ * fit (128 MiB holds e.g. [1, 24, 4608, 128], 69 MB, and [2, 32/8, 8192, 128], 103 MB).  Every
  * call on a GPU shares that GPU's array: calls that overlap on one GPU (different streams or threads without
  * ordering) race and give wrong outputs without an error; calls ordered on one stream do not.  Nothing in the array
  * needs clearing between calls.  The first call on each GPU looks up the array's address (hipGetSymbolAddress, which

@@ -294,7 +294,9 @@ def attention(q8, qs, k8, ks, v8, vs, seq_kv: int, causal: bool = False, block_n
     after that tile (the kernel's seed; without a mask that is tile 0), stored as
     (m_c, l_c, fp16(O_c / l_c)) and merged with M = max m_c, W_c = exp2((m_c - M) * cl) * l_c, L = sum W_c,
     O = sum W_c * fp16(O_c / l_c) (float32, chunk order), then the usual epilogue with L.  A range in which a row
-    sees no key (l_c = 0, m_c = -inf) stores 0 and weighs 0.
+    sees no key (l_c = 0, m_c = -inf) stores 0 and weighs 0.  Plans whose partials the kernel stores in fp32
+    (``fp32_partials``) skip the fp16 rounding.  Causal calls without a mask: a row's later ranges start from the
+    max after tile 0 only where the first row of its 32-row group sees all of that tile.
 
     ``attn_mask``: bool array broadcastable to [B, H, Sq, seq_kv], True where the query attends the key (the
     convention of torch SDPA's boolean masks; no counterpart in the reference's kernel, which sends masked calls to
@@ -347,13 +349,13 @@ def attention(q8, qs, k8, ks, v8, vs, seq_kv: int, causal: bool = False, block_n
     if kv_split is not None:
         chunks, rows = kv_split
         # the kernel's seed: a range that starts after the first kernel tile its 128-row block visits starts from the
-        # walk's running max after that tile, instead of from -inf (no mask: tile 0; the kernel splits only
-        # non-causal calls without a mask, and masked calls with the causal flag folded into the mask)
+        # walk's running max after that tile, instead of from -inf (no mask: tile 0)
+        fp32 = fp32_partials(rows, chunks, seq_kv, D, causal and attn_mask is None)
         first, m_seed = _seed_tiles(q8, cl, k8, ks, v8, seq_kv, causal, block_n, threshold, attn_mask, qpos, wide)
         parts = []
         for c in range(chunks):
             lo = c * k_tiles // chunks
-            m_init = None if first is None else np.where(lo > first, m_seed, F32(-np.inf)).astype(F32)
+            m_init = np.where(lo > first, m_seed, F32(-np.inf)).astype(F32)
             parts.append(_online_softmax(q8, cl, k8, ks, v8, seq_kv, causal, block_n, threshold, *krange(c, chunks),
                                          attn_mask, qpos, wide, m_init=m_init))
         mm = parts[0][1]
@@ -369,7 +371,9 @@ def attention(q8, qs, k8, ks, v8, vs, seq_kv: int, causal: bool = False, block_n
             with np.errstate(divide="ignore", invalid="ignore", over="ignore"):
                 ls = np.where(lc < F32(2.0 ** -64), F32(2.0 ** 64), F32(1.0)).astype(F32)
                 rl = np.where(lc > 0, (F32(1.0) / (lc * ls).astype(F32)).astype(F32), F32(0.0)).astype(F32)
-                pn = ((oc * ls[..., None]).astype(F32) * rl[..., None]).astype(F32).astype(np.float16).astype(F32)
+                pn = ((oc * ls[..., None]).astype(F32) * rl[..., None]).astype(F32)
+                if not fp32:
+                    pn = pn.astype(np.float16).astype(F32)
                 w = np.where(lc > 0, (np.exp2(((mc - mm).astype(F32) * cl).astype(F32)).astype(F32) * lc).astype(F32),
                              F32(0.0)).astype(F32)
             ll = (ll + w).astype(F32)
@@ -388,16 +392,18 @@ def attention(q8, qs, k8, ks, v8, vs, seq_kv: int, causal: bool = False, block_n
 
 def _seed_tiles(q8, cl, k8, ks, v8, seq_kv, causal, block_n, threshold, attn_mask, qpos, wide):
     """Per row: the first 64-key kernel tile that any row of its 128-row block sees (int [B, H, Sq]; a block that
-    sees no key gets a tile past the last), and the walk's running max after that tile.  (None, None) for a causal
-    call without a mask, which the kernel never splits."""
+    sees no key gets a tile past the last), and the walk's running max after that tile.  A causal call without a mask
+    seeds from tile 0 the rows of the 32-row groups whose first row sees all of it."""
     B, H, Sq = cl.shape
     n_tiles = (seq_kv + block_n - 1) // block_n
     per = KERNEL_TILE // block_n
     k_tiles = (seq_kv + KERNEL_TILE - 1) // KERNEL_TILE
     if attn_mask is None:
-        if causal:
-            return None, None
         first = np.zeros((B, H, Sq), dtype=np.int64)
+        if causal:
+            rows, seq_q = qpos
+            group = np.asarray(rows) // 32 * 32
+            first[:, :, group + (seq_kv - seq_q) < KERNEL_TILE - 1] = k_tiles
     else:
         rows, seq_q = qpos
         vis = attn_mask if attn_mask.dtype == bool else attn_mask != -np.inf        # [B, H, Sq, seq_kv]
@@ -597,7 +603,33 @@ def split_rows(B: int, H_total: int, Sq: int, n_full: int, heads=None, block_m: 
     q_tiles = (Sq + block_m - 1) // block_m
     tile = ((np.arange(B)[:, None, None] * H_total + heads[None, :, None]) * q_tiles
             + (np.arange(Sq) // block_m)[None, None, :])
-    return tile >= n_full
+    rows = (tile >= n_full).view(_SplitRows)
+    rows.plan = (B * H_total * q_tiles, n_full)
+    return rows
+
+
+class _SplitRows(np.ndarray):
+    """split_rows' array with the plan it came from, (query tiles, whole tiles), which its slices keep."""
+    plan = None
+
+    def __array_finalize__(self, obj):
+        self.plan = getattr(obj, "plan", None)
+
+
+def fp32_partials(rows, chunks: int, seq_kv: int, head_dim: int, causal: bool) -> bool:
+    """Whether the gfx950 kernel (256 CUs) stores the partials of this plan in fp32: causal plans, and dense plans
+    that split the tiles past a multiple of the CUs rather than those of the last round of resident workgroups.
+    Rows without a plan (a plain bool array) are of the latter kind: fp16."""
+    if causal:
+        return True
+    if getattr(rows, "plan", None) is None:
+        return False
+    n, n_full = rows.plan
+    cus, slots = 256, 256 * {64: 4, 96: 3, 128: 3, 256: 2}[head_dim]
+    rem = n % slots
+    rounds = n <= cus or (rem > 0 and slots // rem >= (4 if n >= 2 * cus else 2) and (seq_kv + 63) // 64 >= 48
+                          and (n >= 2 * cus or 2 * (n % cus) <= cus))
+    return not rounds
 
 
 def round_output(x: np.ndarray, out_dtype: str) -> np.ndarray:

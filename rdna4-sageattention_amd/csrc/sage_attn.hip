@@ -40,6 +40,8 @@
 //   * O^T accumulators (D/32 blocks of 32 channels) give lane l the same query as its S values: m, l and the
 //     rescale stay per lane.
 // LDS tiles use a 16-byte-chunk XOR swizzle so the MFMA operand reads are free of bank conflicts.
+#include <type_traits>
+
 #include "sage_common.h"
 #include "sage_host.h"
 
@@ -107,10 +109,14 @@ __host__ __device__ constexpr bool attn_seeded(int da) { return 127 * 127 * da <
 
 constexpr int ATT_MAX_CHUNKS = 16;
 
-// Workspace of a split launch (units = split tiles x chunks): each chunk's O normalised by its own l, as fp16
+// Workspace of a split launch (units = split tiles x chunks): each chunk's O normalised by its own l, as fp16 or fp32
 // [units][128 rows][D] (|O / l| <= 448, the E4M3 range of V8), then (m, l) as float2 [units][128 rows].
-__host__ __device__ constexpr int64_t ws_ml_offset(int64_t units, int D) { return units * ATT_BM * D * 2; }
-__host__ __device__ constexpr int64_t ws_bytes(int64_t units, int D) { return units * ATT_BM * (2 * D + 8); }
+__host__ __device__ constexpr int64_t ws_ml_offset(int64_t units, int D, bool p32) {
+  return units * ATT_BM * D * (p32 ? 4 : 2);
+}
+__host__ __device__ constexpr int64_t ws_bytes(int64_t units, int D, bool p32) {
+  return units * ATT_BM * ((p32 ? 4 : 2) * D + 8);
+}
 
 // Packed variable-length sequences (VARLEN): block i runs tile tiles[i] = (sequence, head, query tile) or exits when
 // its sequence is -1.  Q8 / QS rows are [H][TQ] (TQ = the `Sq` argument), K8 / KS / V8T the padded packed layout
@@ -134,7 +140,7 @@ __global__ __launch_bounds__(ATT_THREADS, attn_occupancy<layout_dim(HD)>()) void
     const int8_t* __restrict__ q8, const float* __restrict__ qs, const int8_t* __restrict__ k8,
     const float* __restrict__ ks, const uint8_t* __restrict__ v8t, const float* __restrict__ vs,
     uint16_t* __restrict__ out, int64_t osb, int64_t oss, int64_t osh, float* __restrict__ lse, int H, int Hkv,
-    int Sq_arg, int Skv_arg, int Skp, int q_tiles, int total, int n_full, int chunks, float* __restrict__ part,
+    int Sq_arg, int Skv_arg, int Skp, int q_tiles, int total, int n_full, int chunks, int p32, float* __restrict__ part,
     float c0, int dout, VarlenTiles vt, MaskTabs mt, const uint32_t* __restrict__ mbits_tab,
     const int* __restrict__ mcls_tab, const int2* __restrict__ mrange_tab, const uint16_t* __restrict__ mbias_tab) {
   static_assert(!(MASK && (CAUSAL || VARLEN)), "the mask variant folds causality into its bits and is dense only");
@@ -170,10 +176,10 @@ __global__ __launch_bounds__(ATT_THREADS, attn_occupancy<layout_dim(HD)>()) void
   constexpr int LPT = KLOADS + VLOADS;  // direct loads per wave and tile
   __shared__ __attribute__((aligned(16))) uint8_t smem[NBUF][TILE];
 
-  // ---- work decode.  Dense: blocks [0, n_full) own whole query tiles (XCD-grouped); each later block owns one of
-  // the `chunks` key ranges of a split tile.  VARLEN: the tile table. ----
+  // ---- work decode.  Dense: blocks [0, n_full) own whole query tiles (XCD-grouped; causal: longest first); each
+  // later block owns one of the `chunks` key ranges of a split tile.  VARLEN: the tile table. ----
   const bool split = !VARLEN && (int)blockIdx.x >= n_full;
-  int b, h, qt, unit = 0, Sq = Sq_arg, Skv = Skv_arg;
+  int b, h, qt, unit = 0, chunk = 0, Sq = Sq_arg, Skv = Skv_arg;
   int64_t qrow0;       // Q8 / QS row of query 0 of this (sequence, head)
   int khead, kofs;     // K8 / KS / V8T head index and the sequence's first key row inside it
   uint16_t* obase;
@@ -193,13 +199,20 @@ __global__ __launch_bounds__(ATT_THREADS, attn_occupancy<layout_dim(HD)>()) void
   } else {
     int bh;
     if (CAUSAL) {
-      causal_tile(blockIdx.x, total / q_tiles, q_tiles, bh, qt);  // causal launches are never split
+      int tile = blockIdx.x;
+      if (split) {
+        split_unit(blockIdx.x - n_full, total - n_full, chunks, tile, chunk);
+        unit = tile * chunks + chunk;
+        tile += n_full;
+      }
+      causal_tile(tile, total / q_tiles, q_tiles, bh, qt);
     } else {
       int logical;
       if (!split) {
         logical = xcd_remap(blockIdx.x, n_full);
       } else {
         unit = blockIdx.x - n_full;
+        chunk = unit % chunks;
         logical = n_full + unit / chunks;
       }
       bh = logical / q_tiles;
@@ -270,10 +283,10 @@ __global__ __launch_bounds__(ATT_THREADS, attn_occupancy<layout_dim(HD)>()) void
   if (CAUSAL) kv_end = max(0, min(Skv, qt * ATT_BM + ATT_BM + off));  // 0: no row of the tile sees a key
   const int ntiles = (kv_end + BN - 1) / BN;
   int t_lo = 0, t_hi = ntiles;
-  if (split) {
-    const int ch = unit % chunks;
-    t_lo = ch * ntiles / chunks;
-    t_hi = (ch + 1) * ntiles / chunks;
+  if (split) {  // ranges of all the keys; a causal tile may end before its last ranges, which are then empty
+    const int nt = (Skv + BN - 1) / BN;
+    t_lo = chunk * nt / chunks;
+    t_hi = min((chunk + 1) * nt / chunks, ntiles);
   }
 
   // ---- mask: this lane's bit row and this wave's class row; the workgroup runs only the tiles from the first to the
@@ -616,8 +629,9 @@ __global__ __launch_bounds__(ATT_THREADS, attn_occupancy<layout_dim(HD)>()) void
   // reference's max almost never moves after its first tile, so the range then forms the same probabilities, E4M3
   // bytes and rescale decisions as the reference's walk (make_sage_r2.py:141-253) and its merge weight is l alone.
   // The first tile's K goes into the buffer the loop fills last (free until the loop's first prefetch), beside the
-  // range's first tile(s); the dense split tiles are non-causal and unmasked and have at least 4 full key tiles.
-  const bool seed_split = !MASK && !VARLEN && split && t_lo > 0;
+  // range's first tile(s).  Dense launches split only tiles of at least 8 key tiles, so without the causal flag every
+  // row sees the whole first tile; a causal wave whose first row does not starts from -inf.
+  const bool seed_split = !MASK && !VARLEN && split && t_lo > 0 && t_lo < t_hi;
   constexpr int SEED_BUF_OFS = NBUF - 1;  // buffer (t_lo + NBUF - 1) % NBUF
   if (seed_split) {
     const int8_t* kb_ = kbase;
@@ -707,9 +721,11 @@ __global__ __launch_bounds__(ATT_THREADS, attn_occupancy<layout_dim(HD)>()) void
     halves_split_f32(bmh, bm0, bm1);
     // from m = -inf block 0 always sets the max (its keys are all visible); block 1 moves it by the lazy rule
     const float mc1 = fmaxf(bm0, bm1);
-    m = (mc1 - bm0) * cl > 8.0f ? mc1 : bm0;
-    negm = 0.0f - cl * m;
-    if (SPEC_OK) fastok = true;
+    if (!CAUSAL || q0 + off >= BN - 1) {  // wave-uniform
+      m = (mc1 - bm0) * cl > 8.0f ? mc1 : bm0;
+      negm = 0.0f - cl * m;
+      if (SPEC_OK) fastok = true;
+    }
   }
   if (two_ahead)
     wait_vmcnt<LPT>();
@@ -817,18 +833,32 @@ __global__ __launch_bounds__(ATT_THREADS, attn_occupancy<layout_dim(HD)>()) void
     // reciprocal, which then stays finite; l and O of order 1 and above are used as they are.
     const float ls = lt < 0x1p-64f ? 0x1p64f : 1.0f;
     const float rl = lt > 0.0f ? 1.0f / (lt * ls) : 0.0f;  // a range in which the row sees no key stores 0
-    uint16_t* po = reinterpret_cast<uint16_t*>(part) + ((int64_t)unit * ATT_BM + q) * D;
+    if (p32) {
+      float* po = part + ((int64_t)unit * ATT_BM + q) * D;
 #pragma unroll
-    for (int i = 0; i < NPV; ++i)
+      for (int i = 0; i < NPV; ++i)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const uint32_t h0 = f32_to_f16_bits((o[i][4 * g + 0] * ls) * rl), h1 = f32_to_f16_bits((o[i][4 * g + 1] * ls) * rl);
-        const uint32_t h2 = f32_to_f16_bits((o[i][4 * g + 2] * ls) * rl), h3 = f32_to_f16_bits((o[i][4 * g + 3] * ls) * rl);
-        *reinterpret_cast<uint2*>(po + 32 * i + 8 * g + 4 * hf) = make_uint2(h0 | (h1 << 16), h2 | (h3 << 16));
-      }
+        for (int g = 0; g < 4; ++g) {
+          v4f e;
+#pragma unroll
+          for (int u = 0; u < 4; ++u) e[u] = (o[i][4 * g + u] * ls) * rl;
+          *reinterpret_cast<v4f*>(po + 32 * i + 8 * g + 4 * hf) = e;
+        }
+    } else {
+      uint16_t* po = reinterpret_cast<uint16_t*>(part) + ((int64_t)unit * ATT_BM + q) * D;
+#pragma unroll
+      for (int i = 0; i < NPV; ++i)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          uint32_t e[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) e[u] = f32_to_f16_bits((o[i][4 * g + u] * ls) * rl);
+          *reinterpret_cast<uint2*>(po + 32 * i + 8 * g + 4 * hf) = make_uint2(e[0] | (e[1] << 16), e[2] | (e[3] << 16));
+        }
+    }
     const int64_t units = (int64_t)(total - n_full) * chunks;
     if (hf == 0)
-      reinterpret_cast<float2*>(reinterpret_cast<uint8_t*>(part) + ws_ml_offset(units, D))[(int64_t)unit * ATT_BM + q] =
+      reinterpret_cast<float2*>(reinterpret_cast<uint8_t*>(part) + ws_ml_offset(units, D, p32 != 0))[(int64_t)unit * ATT_BM + q] =
           make_float2(m * SSCALE, lt);  // m in S * ks units, as the merge kernel's cl expects
     return;
   }
@@ -868,42 +898,44 @@ __global__ __launch_bounds__(ATT_THREADS, attn_occupancy<layout_dim(HD)>()) void
 // Merge of split tiles: one thread per (split tile s, row r, 4-channel group c), consecutive threads on consecutive
 // groups of a row, so partial reads and output writes are contiguous; every partial load of a thread is issued before
 // the first is used.  With M = max_i m_i over the chunks, W_i = 2^((m_i - M) * cl) * l_i, L = sum_i W_i and
-// O = sum_i W_i * fp16(O_i / l_i) (float32, chunk order), the output is (O * ((1/448) / L)) * VS and
+// O = sum_i W_i * (O_i / l_i) as stored, fp32 with P32 and fp16 otherwise (float32, chunk order), the output is (O * ((1/448) / L)) * VS and
 // lse = ln2 * (cl * M + log2 L), the epilogue of an unsplit tile.  grid = n_split * 128 * (D / 4) / 256 blocks of 256 threads.
 // ------------------------------------------------------------------------------------------------------------------
-template <int D, int OUT_DT>
+template <int D, int OUT_DT, bool P32>
 __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict__ part, const float* __restrict__ qs,
                                                          const float* __restrict__ vs, uint16_t* __restrict__ out,
                                                          int64_t osb, int64_t oss, int64_t osh,
                                                          float* __restrict__ lse, int H, int Hkv, int Sq, int q_tiles,
-                                                         int n_full, int n_split, int chunks, float c0, int dout) {
+                                                         int n_full, int n_split, int chunks, int causal, float c0,
+                                                         int dout) {
   constexpr int NG = D / 4;
   const int idx = blockIdx.x * 256 + threadIdx.x;
   const int cg = idx % NG;
   if (4 * cg >= dout) return;  // head_dim 96: padding channels
   const int q = (idx / NG) % ATT_BM;
   const int s = idx / (NG * ATT_BM);
-  const int logical = n_full + s;
-  const int bh = logical / q_tiles, qt = logical % q_tiles;
+  int bh = (n_full + s) / q_tiles, qt = (n_full + s) % q_tiles;
+  if (causal) causal_tile(n_full + s, (n_full + n_split) / q_tiles, q_tiles, bh, qt);
   const int qrow = qt * ATT_BM + q;
   if (qrow >= Sq) return;
   const int b = bh / H, h = bh % H;
   const int bhk = b * Hkv + h / (H / Hkv);
   const int64_t units = (int64_t)n_split * chunks, unit0 = (int64_t)s * chunks;
   const float2* ml =
-      reinterpret_cast<const float2*>(reinterpret_cast<const uint8_t*>(part) + ws_ml_offset(units, D)) + unit0 * ATT_BM + q;
-  const uint16_t* po = reinterpret_cast<const uint16_t*>(part) + (unit0 * ATT_BM + q) * D + 4 * cg;
+      reinterpret_cast<const float2*>(reinterpret_cast<const uint8_t*>(part) + ws_ml_offset(units, D, P32)) + unit0 * ATT_BM + q;
+  using Part = std::conditional_t<P32, v4f, uint2>;  // the partial of 4 channels
+  const uint8_t* po = reinterpret_cast<const uint8_t*>(part) + ((unit0 * ATT_BM + q) * D + 4 * cg) * (P32 ? 4 : 2);
   // the row's Q scale and the group's V scales first, so that every load of the thread is in flight at once (loaded
   // after the merge arithmetic, the V scales cost a second round trip)
   const float qsr = qs[(int64_t)bh * Sq + qrow];
   const v4f sc4 = *reinterpret_cast<const v4f*>(vs + (int64_t)bhk * D + 4 * cg);
   float2 e[ATT_MAX_CHUNKS];
-  uint2 oi[ATT_MAX_CHUNKS];
+  Part oi[ATT_MAX_CHUNKS];
 #pragma unroll
   for (int i = 0; i < ATT_MAX_CHUNKS; ++i) {
     if (i < chunks) {
       e[i] = ml[i * ATT_BM];
-      oi[i] = *reinterpret_cast<const uint2*>(po + (int64_t)i * ATT_BM * D);
+      oi[i] = *reinterpret_cast<const Part*>(po + (int64_t)i * ATT_BM * D * (P32 ? 4 : 2));
     }
   }
   const float cl = c0 * qsr;
@@ -919,10 +951,17 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict
       // chunk weight times its l; a range in which the row sees no key (l = 0, m = -inf) weighs 0
       const float w = e[i].y > 0.0f ? __builtin_amdgcn_exp2f((e[i].x - M) * cl) * e[i].y : 0.0f;
       L = L + w;
-      acc.x = acc.x + w * f16_lo(oi[i].x);
-      acc.y = acc.y + w * f16_hi(oi[i].x);
-      acc.z = acc.z + w * f16_lo(oi[i].y);
-      acc.w = acc.w + w * f16_hi(oi[i].y);
+      if constexpr (P32) {
+        acc.x = acc.x + w * oi[i][0];
+        acc.y = acc.y + w * oi[i][1];
+        acc.z = acc.z + w * oi[i][2];
+        acc.w = acc.w + w * oi[i][3];
+      } else {
+        acc.x = acc.x + w * f16_lo(oi[i].x);
+        acc.y = acc.y + w * f16_hi(oi[i].x);
+        acc.z = acc.z + w * f16_lo(oi[i].y);
+        acc.w = acc.w + w * f16_hi(oi[i].y);
+      }
     }
   }
   const float inv = L > 0.0f ? (1.0f / 448.0f) / L : 0.0f;  // a row without any visible key is written as 0
@@ -936,14 +975,34 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict
 }
 
 // ------------------------------------------------------------------------------------------------------------------
-// Work plan.  A launch of n_tiles query tiles runs in rounds of `slots` = CUs x resident workgroups per CU.  When the
-// last round is short (rem = n_tiles mod slots tiles), its tiles run at a fraction of the chip's throughput: the
-// plan splits the key range of those rem tiles into chunks = slots / rem parts (at most 16, at least 4 key tiles
-// each) so that the last round fills the chip again, and a merge kernel combines the parts.  Causal tiles are
-// never split.
+// Work plan.  A launch of n query tiles runs on `cus` CUs, each holding `slots / cus` workgroups (3 at head dims 96 and
+// 128, 4 at 64, 2 at 256); its time follows the CU with the most tiles.  Tiles that would make a short last round
+// have their key range split over `chunks` workgroups (at most 16, at least 4 key tiles each) and a merge kernel
+// combines the parts.  The rules, with attention + merge times in us at L key tiles of 64 (bf16, one MI355X):
+//  * n <= cus: every tile, over slots / n ranges.
+//  * the short last round (n mod slots tiles) leaves at least 3/4 of the slots (n < 2 cus: half) and L >= 48: those
+//    tiles, over slots / (n mod slots) ranges; fp16 partials, the most ranges for the least traffic.  d128, L 72,
+//    n 864 (768 + 96 x 8): 165 against 204 whole; with L < 48 the merge costs more than it gains (d128, L 20, n 288:
+//    42 split, 31 whole; d64, L 14, n 448: 29.5 split, 19.7 whole; d64, L 64, n 1536 over 2 ranges: 176 split, 161
+//    whole).
+//  * else the tiles past the last full multiple of cus, at most cus / 2 of them and L >= 32 (20 past the first
+//    round), over cus / that many ranges: one more unit for every CU instead of one more tile for some.  d64, L 64,
+//    n 640 (512 + 128 x 2): 73 against 86 whole; d128, L 72, n 576: 113 against 122; d128, L 265, n 640: 403 against
+//    442; d256, L 69, n 840 (768 + 72 x 3): 272 against 286; d128, L 72, n 1152 (1024 + 128 x 2): 209 against 218 with
+//    768 + 384 x 2.  Below the line: d128, L 20, n 640: 46 split, 43 whole.  More than cus / 2 tiles: d128, L 72,
+//    n 704: 146 split, 132 whole.
+//  * causal: every tile of launches of at most slots / 2 tiles, the longer the key range the more tiles (L >= n / 4
+//    at 256 CUs); past one tile per CU only where the shortest tile sees at least half the keys (chunked prefill).
+//    d128, 192 tiles of a 700-row chunk against 8192 keys (4 ranges): 80 against 120 whole; 384 tiles, 1500 rows
+//    against 9001 keys (2 ranges): 151 against 153-172; square 8 x 2048 (128 tiles, L 32): 31 against 35; below the
+//    line 16 x 2048 (256 tiles, L 32): 41 split, 36 whole; 8 x 8192 (512 tiles): 138 split, 126 whole.
+// The tiles of the last two rules keep fp32 partials, the precision they would be accumulated in whole.
 // ------------------------------------------------------------------------------------------------------------------
+constexpr int CAUSAL_SPLIT_TILES = 512;  // no device has slots for two ranges of more causal tiles than this
+
 struct AttnPlan {
   int n_tiles, n_full, chunks;
+  bool p32;           // fp32 partials (fp16 otherwise)
   int64_t workspace;  // bytes of partial state
 };
 
@@ -979,30 +1038,63 @@ static int resident_blocks(int* per_cu) {
 template <int HD, bool CAUSAL, int OUT_DT>
 static int make_plan(int B, int H, int Sq, int Skv, AttnPlan* p) {
   constexpr int D = layout_dim(HD);
-  const int q_tiles = (Sq + ATT_BM - 1) / ATT_BM;
-  p->n_tiles = B * H * q_tiles;
-  p->n_full = p->n_tiles;
+  const int n = B * H * ((Sq + ATT_BM - 1) / ATT_BM);
+  p->n_tiles = n;
+  p->n_full = n;
   p->chunks = 1;
+  p->p32 = false;
   p->workspace = 0;
-  if (CAUSAL) return SAGE_OK;
+  if (CAUSAL && n > CAUSAL_SPLIT_TILES) return SAGE_OK;
   int cus = 0, per_cu = 0, rc;
   if ((rc = device_cus(&cus))) return rc;
   if ((rc = resident_blocks<HD, CAUSAL, OUT_DT>(&per_cu))) return rc;
   const int slots = cus * per_cu;
   if (slots <= 0) return SAGE_OK;
-  const int rem = p->n_tiles % slots;
-  if (rem == 0) return SAGE_OK;
   const int kv_tiles = (Skv + ATT_BN - 1) / ATT_BN;
-  const int chunks = min(min(slots / rem, kv_tiles / 4), ATT_MAX_CHUNKS);
+  const int most = min(kv_tiles / 4, ATT_MAX_CHUNKS);
+  int rem = 0, chunks = 1;
+  if (CAUSAL) {
+    if ((int64_t)kv_tiles * cus >= 64 * (int64_t)n && (n <= cus || Skv >= 2 * (int64_t)Sq)) {
+      rem = n;
+      chunks = min(slots / n, most);
+      p->p32 = true;
+    }
+  } else {
+    const int rem_round = n % slots, rem_cu = n % cus;
+    const bool past_one = n >= 2 * cus;  // every CU has at least two tiles
+    if (n <= cus || (rem_round > 0 && slots / rem_round >= (past_one ? 4 : 2) && kv_tiles >= 48 &&
+                     (past_one || 2 * rem_cu <= cus))) {
+      rem = rem_round;
+      chunks = rem > 0 ? min(slots / rem, most) : 1;
+    } else if (rem_cu > 0 && (past_one ? 2 * rem_cu <= cus && kv_tiles >= (n > slots ? 20 : 32)
+                                       : 4 * rem_cu <= cus && kv_tiles >= 48)) {
+      rem = rem_cu;
+      chunks = min(cus / rem, most);
+      p->p32 = true;
+    }
+  }
   if (chunks < 2) return SAGE_OK;
-  p->n_full = p->n_tiles - rem;
+  p->n_full = n - rem;
   p->chunks = chunks;
-  p->workspace = ws_bytes((int64_t)rem * chunks, D);
+  p->workspace = ws_bytes((int64_t)rem * chunks, D, p->p32);
   return SAGE_OK;
 }
 
 // c0 = log2(e) / sqrt(head_dim) with the kernel's built-in sm_scale (other scales are folded into QS)
 static float logit_scale_base(int head_dim) { return (float)((1.0 / __builtin_sqrt((double)head_dim)) * 1.4426950408889634); }
+
+template <int D, int OUT_DT>
+static void launch_merge(const AttnPlan& p, int n_split, const float* part, const float* qs, const float* vs,
+                         uint16_t* out, int64_t osb, int64_t oss, int64_t osh, float* lse, int H, int Hkv, int Sq,
+                         int q_tiles, int causal, float c0, int hd, hipStream_t st) {
+  const dim3 grid(n_split * (ATT_BM * D / 4 / 256));
+  if (p.p32)
+    hipLaunchKernelGGL((attn_merge_kernel<D, OUT_DT, true>), grid, dim3(256), 0, st, part, qs, vs, out, osb, oss, osh,
+                       lse, H, Hkv, Sq, q_tiles, p.n_full, n_split, p.chunks, causal, c0, hd);
+  else
+    hipLaunchKernelGGL((attn_merge_kernel<D, OUT_DT, false>), grid, dim3(256), 0, st, part, qs, vs, out, osb, oss, osh,
+                       lse, H, Hkv, Sq, q_tiles, p.n_full, n_split, p.chunks, causal, c0, hd);
+}
 
 // HD: head dim (64, 96, 128, 256); D = layout_dim(HD) channels of the intermediates (96 runs on the 128-channel
 // layout); hd == HD, the output channels
@@ -1017,6 +1109,7 @@ static int launch_attn(const int8_t* q8, const float* qs, const int8_t* k8, cons
     const int q_tiles = (Sq + ATT_BM - 1) / ATT_BM;
     p.n_tiles = p.n_full = B * H * q_tiles;
     p.chunks = 1;
+    p.p32 = false;
     p.workspace = 0;
   } else {
     if ((rc = make_plan<HD, CAUSAL, OUT_DT>(B, H, Sq, Skv, &p))) return rc;
@@ -1032,11 +1125,10 @@ static int launch_attn(const int8_t* q8, const float* qs, const int8_t* k8, cons
   float* part = static_cast<float*>(workspace);
   hipLaunchKernelGGL((attn_kernel<HD, CAUSAL, OUT_DT, false>), dim3(blocks), dim3(ATT_THREADS), 0, st, q8, qs, k8, ks, v8t,
                      vs, o, osb, oss, osh, lse, H, Hkv, Sq, Skv, kv_pad(Skv), q_tiles, p.n_tiles, p.n_full, p.chunks,
-                     part, c0, hd, VarlenTiles{}, MaskTabs{}, nullptr, nullptr, nullptr, nullptr);
+                     (int)p.p32, part, c0, hd, VarlenTiles{}, MaskTabs{}, nullptr, nullptr, nullptr, nullptr);
   if (n_split > 0) {
     if ((rc = check_launch("attention launch"))) return rc;
-    hipLaunchKernelGGL((attn_merge_kernel<D, OUT_DT>), dim3(n_split * (ATT_BM * D / 4 / 256)), dim3(256), 0, st,
-                       part, qs, vs, o, osb, oss, osh, lse, H, Hkv, Sq, q_tiles, p.n_full, n_split, p.chunks, c0, hd);
+    launch_merge<D, OUT_DT>(p, n_split, part, qs, vs, o, osb, oss, osh, lse, H, Hkv, Sq, q_tiles, CAUSAL, c0, hd, st);
   }
   return check_launch("attention launch");
 }
@@ -1110,7 +1202,7 @@ static int launch_attn_varlen(const int8_t* q8, const float* qs, const int8_t* k
                               int TQ, int TKP, int hd, int n_blocks, VarlenTiles vt, hipStream_t st) {
   hipLaunchKernelGGL((attn_kernel<HD, CAUSAL, OUT_DT, true>), dim3(n_blocks), dim3(ATT_THREADS), 0, st, q8, qs, k8, ks,
                      v8t, vs, static_cast<uint16_t*>(out), (int64_t)0, oss, osh, nullptr, H, Hkv, TQ, 0, TKP, 0,
-                     n_blocks, n_blocks, 1, nullptr, logit_scale_base(hd), hd, vt, MaskTabs{}, nullptr, nullptr,
+                     n_blocks, n_blocks, 1, 0, nullptr, logit_scale_base(hd), hd, vt, MaskTabs{}, nullptr, nullptr,
                      nullptr, nullptr);
   return check_launch("varlen attention launch");
 }
@@ -1157,12 +1249,10 @@ static int launch_attn_mask(const int8_t* q8, const float* qs, const int8_t* k8,
   float* part = static_cast<float*>(workspace);
   hipLaunchKernelGGL((attn_kernel<HD, false, OUT_DT, false, true>), dim3(blocks), dim3(ATT_THREADS), 0, st, q8, qs, k8,
                      ks, v8t, vs, o, osb, oss, osh, nullptr, H, Hkv, Sq, Skv, kv_pad(Skv), q_tiles, p.n_tiles,
-                     p.n_full, p.chunks, part, c0, hd, VarlenTiles{}, mt, mt.bits, mt.cls, mt.range, mt.bias);
+                     p.n_full, p.chunks, (int)p.p32, part, c0, hd, VarlenTiles{}, mt, mt.bits, mt.cls, mt.range, mt.bias);
   if (n_split > 0) {
     if ((rc = check_launch("masked attention launch"))) return rc;
-    hipLaunchKernelGGL((attn_merge_kernel<D, OUT_DT>), dim3(n_split * (ATT_BM * D / 4 / 256)), dim3(256), 0, st,
-                       part, qs, vs, o, osb, oss, osh, nullptr, H, Hkv, Sq, q_tiles, p.n_full, n_split, p.chunks, c0,
-                       hd);
+    launch_merge<D, OUT_DT>(p, n_split, part, qs, vs, o, osb, oss, osh, nullptr, H, Hkv, Sq, q_tiles, 0, c0, hd, st);
   }
   return check_launch("masked attention launch");
 }

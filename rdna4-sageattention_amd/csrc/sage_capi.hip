@@ -43,11 +43,13 @@ int forward_quant_impl(const void*, int64_t, int64_t, int64_t, const void*, int6
                        int64_t, int64_t, int64_t, int, int, int, int, int, int, int, float, int8_t*, float*, float*,
                        int8_t*, float*, uint8_t*, float*, const MaskPrep*, void*);
 
-// sage_forward's workspace: the attention plan's partial state, then (256-byte aligned) the per-chunk V maxima.
-static int forward_workspace(int B, int H, int Hkv, int Sq, int Skv, int D, int causal, int64_t* attn_bytes,
+// sage_forward's workspace: the attention plan's partial state (none without split), then (256-byte aligned) the
+// per-chunk V maxima.
+static int forward_workspace(int B, int H, int Hkv, int Sq, int Skv, int D, int causal, bool split, int64_t* attn_bytes,
                              int64_t* total) {
   int rc = attn_plan_impl(B, H, Sq, Skv, D, causal, nullptr, nullptr, attn_bytes);
   if (rc) return rc;
+  if (!split) *attn_bytes = 0;
   *total = (*attn_bytes + 255) / 256 * 256 + vamax_partial_bytes(B, Hkv, Skv, D);
   return SAGE_OK;
 }
@@ -81,6 +83,48 @@ static int scratch_base(void** base) {
 }
 
 static int64_t align256(int64_t n) { return (n + 255) / 256 * 256; }
+
+// sage_forward's body.  split = false: every attention tile whole, with a workspace of the V maxima alone.
+static int forward_impl(const void* q, int64_t qsb, int64_t qss, int64_t qsh, const void* k, int64_t ksb, int64_t kss,
+                        int64_t ksh, const void* v, int64_t vsb, int64_t vss, int64_t vsh, void* out, int64_t osb,
+                        int64_t oss, int64_t osh, int B, int H, int Hkv, int Sq, int Skv, int D, int dtype, int causal,
+                        float qs_mul, int8_t* q8, float* qs, int8_t* k8, float* ks, uint8_t* v8t, float* vs,
+                        void* workspace, int64_t workspace_bytes, bool split, void* stream) {
+  // validate everything before the first launch so a bad call leaves the stream untouched
+  SAGE_REQUIRE(B > 0 && H > 0 && Hkv > 0 && Sq > 0 && Skv > 0, "sage_forward: sizes must be positive");
+  SAGE_REQUIRE(H % Hkv == 0, "sage_forward: heads %d not a multiple of kv heads %d", H, Hkv);
+  if (!head_dim_ok(D))
+    return fail(SAGE_ERR_UNSUPPORTED, "sage_forward: head_dim %d (supported 64, 96, 128, 256)", D);
+  if (causal && Sq > Skv) return fail(SAGE_ERR_UNSUPPORTED, "sage_forward: causal attention needs q_len <= kv_len");
+  int rc = forward_inputs_check(q, qsb, qss, qsh, k, ksb, kss, ksh, v, vsb, vss, vsh, B, H, Hkv, Sq, Skv, D, dtype,
+                                "sage_forward");
+  if (rc) return rc;
+  if ((rc = check_qs_mul(qs_mul, "sage_forward"))) return rc;
+  // the attention step's checks (its size limits, the output, the intermediates) before the quantizers launch
+  if ((rc = attn_args_check(q8, qs, k8, ks, v8t, vs, out, osb, oss, osh, B, H, Hkv, Sq, Skv, D, causal, dtype,
+                            "sage_forward")))
+    return rc;
+  if (workspace == nullptr) {
+    // no workspace: V maxima by atomics (four quantization launches) and every attention tile whole
+    if ((rc = v_amax_impl(v, vsb, vss, vsh, B, Hkv, Skv, D, dtype, vs, stream))) return rc;
+    if ((rc = quant_q_impl(q, qsb, qss, qsh, B, H, Sq, D, dtype, qs_mul, q8, qs, stream))) return rc;
+    if ((rc = quant_kv_impl(k, ksb, kss, ksh, v, vsb, vss, vsh, B, Hkv, Skv, D, dtype, vs, k8, ks, v8t, stream)))
+      return rc;
+    return attn_impl(q8, qs, k8, ks, v8t, vs, out, osb, oss, osh, B, H, Hkv, Sq, Skv, D, causal, dtype, nullptr,
+                     nullptr, 0, stream);
+  }
+  int64_t attn_bytes = 0, need = 0;
+  if ((rc = forward_workspace(B, H, Hkv, Sq, Skv, D, causal, split, &attn_bytes, &need))) return rc;
+  SAGE_REQUIRE(workspace_bytes >= need, "sage_forward: workspace of %lld bytes, the plan needs %lld",
+               (long long)workspace_bytes, (long long)need);
+  SAGE_REQUIRE(((uintptr_t)workspace & 255u) == 0, "sage_forward: workspace must be 256-byte aligned");
+  float* vpart = reinterpret_cast<float*>(static_cast<char*>(workspace) + (attn_bytes + 255) / 256 * 256);
+  if ((rc = forward_quant_impl(q, qsb, qss, qsh, k, ksb, kss, ksh, v, vsb, vss, vsh, B, H, Hkv, Sq, Skv, D, dtype,
+                               qs_mul, q8, qs, vpart, k8, ks, v8t, vs, nullptr, stream)))
+    return rc;
+  return attn_impl(q8, qs, k8, ks, v8t, vs, out, osb, oss, osh, B, H, Hkv, Sq, Skv, D, causal, dtype, nullptr,
+                   attn_bytes ? workspace : nullptr, attn_bytes, stream);
+}
 
 }  // namespace sage
 
@@ -118,7 +162,7 @@ int sage_forward_workspace(int B, int H, int Hkv, int Sq, int Skv, int D, int ca
   SAGE_REQUIRE(workspace_bytes != nullptr, "sage_forward_workspace: workspace_bytes is NULL");
   SAGE_REQUIRE(Hkv > 0 && H % Hkv == 0, "sage_forward_workspace: heads %d not a multiple of kv heads %d", H, Hkv);
   int64_t attn = 0;
-  return sage::forward_workspace(B, H, Hkv, Sq, Skv, D, causal, &attn, workspace_bytes);
+  return sage::forward_workspace(B, H, Hkv, Sq, Skv, D, causal, true, &attn, workspace_bytes);
 }
 
 int sage_forward(const void* q, int64_t qsb, int64_t qss, int64_t qsh, const void* k, int64_t ksb, int64_t kss,
@@ -127,40 +171,8 @@ int sage_forward(const void* q, int64_t qsb, int64_t qss, int64_t qsh, const voi
                  int8_t* q8, float* qs, int8_t* k8, float* ks, uint8_t* v8t, float* vs, void* workspace,
                  int64_t workspace_bytes, void* stream) {
   sage::clear_error();
-  // validate everything before the first launch so a bad call leaves the stream untouched
-  SAGE_REQUIRE(B > 0 && H > 0 && Hkv > 0 && Sq > 0 && Skv > 0, "sage_forward: sizes must be positive");
-  SAGE_REQUIRE(H % Hkv == 0, "sage_forward: heads %d not a multiple of kv heads %d", H, Hkv);
-  if (!sage::head_dim_ok(D))
-    return sage::fail(SAGE_ERR_UNSUPPORTED, "sage_forward: head_dim %d (supported 64, 96, 128, 256)", D);
-  if (causal && Sq > Skv) return sage::fail(SAGE_ERR_UNSUPPORTED, "sage_forward: causal attention needs q_len <= kv_len");
-  int rc = sage::forward_inputs_check(q, qsb, qss, qsh, k, ksb, kss, ksh, v, vsb, vss, vsh, B, H, Hkv, Sq, Skv, D, dtype,
-                                      "sage_forward");
-  if (rc) return rc;
-  if ((rc = sage::check_qs_mul(qs_mul, "sage_forward"))) return rc;
-  // the attention step's checks (its size limits, the output, the intermediates) before the quantizers launch
-  if ((rc = sage::attn_args_check(q8, qs, k8, ks, v8t, vs, out, osb, oss, osh, B, H, Hkv, Sq, Skv, D, causal, dtype,
-                                  "sage_forward")))
-    return rc;
-  if (workspace == nullptr) {
-    // no workspace: V maxima by atomics (four quantization launches) and every attention tile whole
-    if ((rc = sage::v_amax_impl(v, vsb, vss, vsh, B, Hkv, Skv, D, dtype, vs, stream))) return rc;
-    if ((rc = sage::quant_q_impl(q, qsb, qss, qsh, B, H, Sq, D, dtype, qs_mul, q8, qs, stream))) return rc;
-    if ((rc = sage::quant_kv_impl(k, ksb, kss, ksh, v, vsb, vss, vsh, B, Hkv, Skv, D, dtype, vs, k8, ks, v8t, stream)))
-      return rc;
-    return sage::attn_impl(q8, qs, k8, ks, v8t, vs, out, osb, oss, osh, B, H, Hkv, Sq, Skv, D, causal, dtype, nullptr,
-                           nullptr, 0, stream);
-  }
-  int64_t attn_bytes = 0, need = 0;
-  if ((rc = sage::forward_workspace(B, H, Hkv, Sq, Skv, D, causal, &attn_bytes, &need))) return rc;
-  SAGE_REQUIRE(workspace_bytes >= need, "sage_forward: workspace of %lld bytes, the plan needs %lld",
-               (long long)workspace_bytes, (long long)need);
-  SAGE_REQUIRE(((uintptr_t)workspace & 255u) == 0, "sage_forward: workspace must be 256-byte aligned");
-  float* vpart = reinterpret_cast<float*>(static_cast<char*>(workspace) + (attn_bytes + 255) / 256 * 256);
-  if ((rc = sage::forward_quant_impl(q, qsb, qss, qsh, k, ksb, kss, ksh, v, vsb, vss, vsh, B, H, Hkv, Sq, Skv, D, dtype,
-                                     qs_mul, q8, qs, vpart, k8, ks, v8t, vs, nullptr, stream)))
-    return rc;
-  return sage::attn_impl(q8, qs, k8, ks, v8t, vs, out, osb, oss, osh, B, H, Hkv, Sq, Skv, D, causal, dtype, nullptr,
-                         attn_bytes ? workspace : nullptr, attn_bytes, stream);
+  return sage::forward_impl(q, qsb, qss, qsh, k, ksb, kss, ksh, v, vsb, vss, vsh, out, osb, oss, osh, B, H, Hkv, Sq, Skv,
+                            D, dtype, causal, qs_mul, q8, qs, k8, ks, v8t, vs, workspace, workspace_bytes, true, stream);
 }
 
 int sage_forward_noalloc(const void* q, int64_t qsb, int64_t qss, int64_t qsh, const void* k, int64_t ksb,
@@ -179,7 +191,7 @@ int sage_forward_noalloc(const void* q, int64_t qsb, int64_t qss, int64_t qsh, c
   const int64_t dl = sage::layout_dim(D), skp = sage::kv_pad(Skv);
   const int64_t nq = (int64_t)B * H * Sq, nkv = (int64_t)B * Hkv;
   int64_t attn_bytes = 0, ws_bytes = 0;
-  if ((rc = sage::forward_workspace(B, H, Hkv, Sq, Skv, D, causal, &attn_bytes, &ws_bytes))) return rc;
+  if ((rc = sage::forward_workspace(B, H, Hkv, Sq, Skv, D, causal, true, &attn_bytes, &ws_bytes))) return rc;
   const int64_t o_q8 = 0;
   const int64_t o_qs = o_q8 + sage::align256(nq * dl);
   const int64_t o_k8 = o_qs + sage::align256(nq * 4);
@@ -187,6 +199,9 @@ int sage_forward_noalloc(const void* q, int64_t qsb, int64_t qss, int64_t qsh, c
   const int64_t o_v8t = o_ks + sage::align256(nkv * (skp / SAGE_KV_BLOCK) * 4);
   const int64_t o_vs = o_v8t + sage::align256(nkv * dl * skp);
   const int64_t o_ws = o_vs + sage::align256(nkv * dl * 4);
+  // where only the split tiles' partials do not fit, every tile runs whole
+  const bool split = o_ws + ws_bytes <= (int64_t)SAGE_NOALLOC_SCRATCH_BYTES;
+  if (!split && (rc = sage::forward_workspace(B, H, Hkv, Sq, Skv, D, causal, false, &attn_bytes, &ws_bytes))) return rc;
   const int64_t need = o_ws + ws_bytes;
   if (need > (int64_t)SAGE_NOALLOC_SCRATCH_BYTES)
     return sage::fail(SAGE_ERR_INVALID, "%s: this shape needs %lld bytes of scratch, the library holds %lld "
@@ -195,10 +210,11 @@ int sage_forward_noalloc(const void* q, int64_t qsb, int64_t qss, int64_t qsh, c
   void* base = nullptr;
   if ((rc = sage::scratch_base(&base))) return rc;
   uint8_t* p = static_cast<uint8_t*>(base);
-  return sage_forward(q, qsb, qss, qsh, k, ksb, kss, ksh, v, vsb, vss, vsh, out, osb, oss, osh, B, H, Hkv, Sq, Skv, D,
-                      dtype, causal, qs_mul, reinterpret_cast<int8_t*>(p + o_q8), reinterpret_cast<float*>(p + o_qs),
-                      reinterpret_cast<int8_t*>(p + o_k8), reinterpret_cast<float*>(p + o_ks), p + o_v8t,
-                      reinterpret_cast<float*>(p + o_vs), p + o_ws, ws_bytes, stream);
+  return sage::forward_impl(q, qsb, qss, qsh, k, ksb, kss, ksh, v, vsb, vss, vsh, out, osb, oss, osh, B, H, Hkv, Sq, Skv,
+                            D, dtype, causal, qs_mul, reinterpret_cast<int8_t*>(p + o_q8),
+                            reinterpret_cast<float*>(p + o_qs), reinterpret_cast<int8_t*>(p + o_k8),
+                            reinterpret_cast<float*>(p + o_ks), p + o_v8t, reinterpret_cast<float*>(p + o_vs), p + o_ws,
+                            ws_bytes, split, stream);
 }
 
 }  // extern "C"

@@ -247,4 +247,18 @@ __device__ __forceinline__ void causal_tile(int id, int bh_count, int q_tiles, i
   }
 }
 
+// The tile and key range of workgroup `id` among `tiles` split tiles of `chunks` ranges each: the ranges of one tile
+// on one XCD (they read the same Q and write the same partials' neighbours) where the tiles divide over the 8.
+__device__ __forceinline__ void split_unit(int id, int tiles, int chunks, int& tile, int& chunk) {
+  constexpr int NX = 8;
+  if (tiles % NX == 0) {
+    const int x = id % NX, i = id / NX;
+    chunk = i % chunks;
+    tile = i / chunks * NX + x;
+  } else {
+    chunk = id % chunks;
+    tile = id / chunks;
+  }
+}
+
 }  // namespace sage
