@@ -58,8 +58,9 @@ template <int ROW_BYTES> __device__ __forceinline__ int swz(int row, int chunk) 
   return chunk ^ ((row >> 2) & 3);
 }
 
-// workgroups per CU the launch bounds ask for: d256 tiles take 64 KiB of LDS and twice the accumulators
-template <int D> constexpr int attn_occupancy() { return D == 256 ? 2 : 3; }
+// workgroups per CU the launch bounds ask for: d256 tiles take 64 KiB of LDS and twice the accumulators; d64 reaches 4
+// by itself except with an additive mask (129 VGPRs, one too many, without the bound)
+template <int D, bool ADDITIVE> constexpr int attn_occupancy() { return D == 256 ? 2 : D == 64 && ADDITIVE ? 4 : 3; }
 
 // Direct global -> LDS copy of 16 bytes per lane: the data lands at LDS address (M0 base) + 16 * lane, so a wave
 // writes one contiguous KiB; `lds` must be wave-uniform.
@@ -68,15 +69,18 @@ __device__ __forceinline__ void copy16_to_lds(const void* g, void* lds) {
                                    (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
 }
 
+// The lane's index, computed anew where it is rarely needed (kept from the kernel's start it would hold a register
+// through the tile loops)
+__device__ __forceinline__ int lane_id() {
+  int l;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(l));
+  return l;
+}
+
 // 32-bit load through the global address space (a generic pointer would give a flat load, which also counts on the
 // LDS counter, so every LDS wait of the tile would wait for it)
 __device__ __forceinline__ uint32_t load_global_u32(const uint8_t* p) {
   return *(const __attribute__((address_space(1))) uint32_t*)(p);
-}
-
-// 16 bytes through the global address space
-__device__ __forceinline__ v4i load_global_v4i(const uint8_t* p) {
-  return *(const __attribute__((address_space(1))) v4i*)(p);
 }
 
 // an additive mask element (the input dtype's 16 bits in the low half) as fp32
@@ -134,15 +138,18 @@ struct VarlenTiles {
 // rows are zero-padded) and DA = HD the channels the MFMAs cover: the zero channels of head_dim 96 add nothing to S
 // and give output channels that are not written, so its tiles run 3 of the 4 QK and PV MFMA blocks of the 128-channel
 // layout.  `dout` output channels are written.  c0 = log2(e) / sqrt(head_dim).
-// MASK: a boolean mask (MaskTabs) instead of the causal / padding bound; the causal flag is folded into its bits.
-template <int HD, bool CAUSAL, int OUT_DT, bool VARLEN, bool MASK = false>
-__global__ __launch_bounds__(ATT_THREADS, attn_occupancy<layout_dim(HD)>()) void attn_kernel(
+// MASK: a mask (MaskTabs) instead of the causal / padding bound, whose causal flag is folded into its bits: MASK_BOOL
+// (classes 0-2) or MASK_ADD (additive, class 3 as well; apart because its tile body costs the other bodies registers).
+constexpr int MASK_NONE = 0, MASK_BOOL = 1, MASK_ADD = 2;
+constexpr int64_t MASK_ROW_32BIT = 1 << 26;  // 31 rows of at most this many 16-bit elements: a 32-bit byte offset
+template <int HD, bool CAUSAL, int OUT_DT, bool VARLEN, int MASK = MASK_NONE>
+__global__ __launch_bounds__(ATT_THREADS, (attn_occupancy<layout_dim(HD), MASK == MASK_ADD>())) void attn_kernel(
     const int8_t* __restrict__ q8, const float* __restrict__ qs, const int8_t* __restrict__ k8,
     const float* __restrict__ ks, const uint8_t* __restrict__ v8t, const float* __restrict__ vs,
     uint16_t* __restrict__ out, int64_t osb, int64_t oss, int64_t osh, float* __restrict__ lse, int H, int Hkv,
     int Sq_arg, int Skv_arg, int Skp, int q_tiles, int total, int n_full, int chunks, int p32, float* __restrict__ part,
     float c0, int dout, VarlenTiles vt, MaskTabs mt, const uint32_t* __restrict__ mbits_tab,
-    const int* __restrict__ mcls_tab, const int2* __restrict__ mrange_tab, const uint16_t* __restrict__ mbias_tab) {
+    const int* __restrict__ mcls_tab, const int2* __restrict__ mrange_tab) {
   static_assert(!(MASK && (CAUSAL || VARLEN)), "the mask variant folds causality into its bits and is dense only");
   constexpr int D = layout_dim(HD);
   constexpr int DA = HD;
@@ -294,16 +301,17 @@ __global__ __launch_bounds__(ATT_THREADS, attn_occupancy<layout_dim(HD)>()) void
   // exactly the online softmax over them) ----
   const uint8_t* mbase = nullptr;  // this (batch, head)'s mask words; the lane's row at byte offset moff
   uint32_t moff = 0;                 // (a (batch, head) slice of the bits is below 2 GiB, checked on the host)
-  const uint8_t* bbase = nullptr;  // the same for the bias values of an additive mask (64 bytes per word)
-  uint32_t boff = 0;
+  const uint8_t* braw = nullptr;  // an additive mask: the values of the wave's first row; the lane's row and first
+  uint32_t boff = 0;              // 16-byte chunk at byte offset boff (row strides up to MASK_ROW_32BIT)
   const int* mcls = nullptr;
   int mseed_tile = -1;  // MASK: the tile whose full pass seeds a split range's running max (-1: none)
   if (MASK) {
     const int64_t wslice = (int64_t)b * mt.bsb + (int64_t)h * mt.bsh;
     mbase = reinterpret_cast<const uint8_t*>(mbits_tab + wslice);
     moff = (uint32_t)(((int64_t)qr * mt.bsq + hf) * 4);
-    bbase = reinterpret_cast<const uint8_t*>(mbias_tab + wslice * 32);
-    boff = (uint32_t)(((int64_t)qr * mt.bsq + hf) * 64);
+    const int qw = min(q0, Sq - 1);
+    braw = reinterpret_cast<const uint8_t*>(mt.raw + (b * mt.vsb + h * mt.vsh + qw * mt.vsq));
+    boff = (uint32_t)(((qr - qw) * mt.vsq + 8 * hf) * 2);
     mcls = mcls_tab + (int64_t)b * mt.csb + (int64_t)h * mt.csh + (int64_t)min(q0 >> 5, mt.groups - 1) * mt.csg;
     const int2 r = mrange_tab[(int64_t)b * mt.rsb + (int64_t)h * mt.rsh + min(qt, mt.rblocks - 1)];
     // a split range after the block's first visited tile starts from the walk's max after that tile (below)
@@ -347,6 +355,29 @@ __global__ __launch_bounds__(ATT_THREADS, attn_occupancy<layout_dim(HD)>()) void
     _Pragma("unroll") for (int j_ = 0; j_ < VLOADS; ++j_) {                                                \
       asm volatile("" : "+v"(voff[j_]));                                                                 \
       copy16_to_lds(vb_ + voff[j_], dst_ + KTILE + (wave * VLOADS + j_) * 1024);                            \
+    }                                                                                                      \
+  } while (0)
+
+  // The lane's bias values of tile T (class 3): four 16-byte chunks, keys [64 T + 16 i + 8 hf, + 8), of its row of the
+  // mask, or of the copy of a partial last tile.  The tile body turns them into accumulator order.  Both tests are
+  // wave-uniform; the second one's rows are so far apart that a lane's offset takes 64 bits.
+#define SAGE_LOAD_BIAS(T, BW)                                                                              \
+  do {                                                                                                     \
+    const uint8_t* p_ = braw + 128 * (int64_t)(T);                                                         \
+    uint32_t o_ = boff;                                                                                    \
+    const bool part_ = ((T) + 1) * BN > Skv;                                                               \
+    if (part_) {                                                                                           \
+      const int ql_ = lane_id(), qw_ = min(q0, Sq - 1);                                                    \
+      p_ = reinterpret_cast<const uint8_t*>(mt.bias + (b * mt.psb + h * mt.psh + qw_ * mt.psq));           \
+      o_ = (uint32_t)(((min(q0 + (ql_ & 31), Sq - 1) - qw_) * (int)mt.psq + 8 * (ql_ >> 5)) * 2);          \
+    }                                                                                                      \
+    asm volatile("" : "+s"(p_), "+v"(o_));                                                                 \
+    if (mt.vsq > MASK_ROW_32BIT && !part_) {                                                               \
+      const int ql_ = lane_id(), qw_ = min(q0, Sq - 1);                                                    \
+      const uint8_t* r_ = p_ + ((min(q0 + (ql_ & 31), Sq - 1) - qw_) * mt.vsq + 8 * (ql_ >> 5)) * 2;       \
+      _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) (BW)[i_] = load16_2aligned(r_ + 32 * i_);           \
+    } else {                                                                                               \
+      _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) (BW)[i_] = load16_2aligned(p_ + o_ + 32 * i_);      \
     }                                                                                                      \
   } while (0)
 
@@ -454,14 +485,32 @@ __global__ __launch_bounds__(ATT_THREADS, attn_occupancy<layout_dim(HD)>()) void
             _Pragma("unroll") for (int v_ = 0; v_ < 16; ++v_) sf_[kb_][v_] -= SEED_F;                      \
         }                                                                                                  \
         float tm0_ = -INFINITY, tm1_ = -INFINITY;                                                          \
-        _Pragma("unroll") for (int kb_ = 0; kb_ < 2; ++kb_)                                                \
-          _Pragma("unroll") for (int v_ = 0; v_ < 16; ++v_) {                                              \
-            const uint32_t bw_ = (BW)[(16 * kb_ + v_) >> 3][((16 * kb_ + v_) >> 1) & 3];                   \
-            const float b_ = mask_half_to_f32<OUT_DT>((v_ & 1) ? (bw_ >> 16) : (bw_ & 0xFFFFu));           \
-            const float in_ = __builtin_fmaf(b_, 1.44269504088896341f, kb_ ? ns1_ : ns0_);                 \
-            sf_[kb_][v_] = __builtin_fmaf(sf_[kb_][v_], kb_ ? ct1_ : ct0_, in_);                           \
-            if (kb_) tm1_ = fmaxf(tm1_, sf_[kb_][v_]);                                                     \
-            else tm0_ = fmaxf(tm0_, sf_[kb_][v_]);                                                         \
+        if (mt.causal && t_ * BN + BN - 1 > q0 + off) {  /* the tile crosses a row's diagonal (wave-uniform) */ \
+          const int ql_ = lane_id();                                                                       \
+          const int lim_ = min(q0 + (ql_ & 31), Sq - 1) + off - (t_ * BN + 8 * (ql_ >> 5));                \
+          constexpr uint32_t ninf_ = OUT_DT == DT_BF16 ? 0xFF80u : 0xFC00u;                                \
+          _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_)                                                 \
+            _Pragma("unroll") for (int d_ = 0; d_ < 4; ++d_) {                                             \
+              uint32_t w_ = (uint32_t)(BW)[i_][d_];                                                        \
+              if (16 * i_ + 2 * d_ > lim_) w_ = (w_ & 0xFFFF0000u) | ninf_;                                \
+              if (16 * i_ + 2 * d_ + 1 > lim_) w_ = (w_ & 0xFFFFu) | (ninf_ << 16);                        \
+              (BW)[i_][d_] = (int)w_;                                                                      \
+            }                                                                                              \
+        }                                                                                                  \
+        /* the lane's keys of the 16 that two neighbouring chunks hold: its half of the row's other lane's chunk \
+           comes over by one swap per pair of words */                                                     \
+        _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_)                                                   \
+          _Pragma("unroll") for (int d_ = 0; d_ < 2; ++d_) {                                               \
+            const auto x_ = __builtin_amdgcn_permlane32_swap((BW)[i_][d_], (BW)[i_][d_ + 2], false, false); \
+            _Pragma("unroll") for (int c_ = 0; c_ < 2; ++c_)                                               \
+              _Pragma("unroll") for (int e_ = 0; e_ < 2; ++e_) {                                           \
+                const int kb_ = i_ >> 1, v_ = 8 * (i_ & 1) + 4 * c_ + 2 * d_ + e_;                         \
+                const float b_ = mask_half_to_f32<OUT_DT>(e_ ? (x_[c_] >> 16) : (x_[c_] & 0xFFFFu));       \
+                const float in_ = __builtin_fmaf(b_, 1.44269504088896341f, kb_ ? ns1_ : ns0_);             \
+                sf_[kb_][v_] = __builtin_fmaf(sf_[kb_][v_], kb_ ? ct1_ : ct0_, in_);                       \
+                if (kb_) tm1_ = fmaxf(tm1_, sf_[kb_][v_]);                                                 \
+                else tm0_ = fmaxf(tm0_, sf_[kb_][v_]);                                                     \
+              }                                                                                            \
           }                                                                                                \
         bmh_ = halves_max_f32(tm0_, tm1_);                                                                 \
       } else {                                                                                             \
@@ -657,10 +706,9 @@ __global__ __launch_bounds__(ATT_THREADS, attn_occupancy<layout_dim(HD)>()) void
     } else if (cs == 2) {
       const uint32_t mw = load_global_u32(mbase + (moff + 8u * (uint32_t)ts));
       SAGE_TILE_PASSES(ts, 2, mw, bw_none, wide);
-    } else if (cs == 3) {
+    } else if (MASK == MASK_ADD && cs == 3) {
       v4i bias_w[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) bias_w[i] = load_global_v4i(bbase + (boff + 128u * (uint32_t)ts + 16u * i));
+      SAGE_LOAD_BIAS(ts, bias_w);
       SAGE_TILE_PASSES(ts, 3, 0u, bias_w, wide);
     }
     l = 0.0f;
@@ -776,12 +824,9 @@ __global__ __launch_bounds__(ATT_THREADS, attn_occupancy<layout_dim(HD)>()) void
       // a run of class 3 (additive mask): the lane's 64 bytes of bias values of the tile are loaded before the next
       // tile's direct loads, which are always issued here (the last iteration reloads its own tile into the idle
       // buffer), so the wait for the values counts the direct loads behind them and does not wait for them
-      for (; t < t_hi && c_nxt == 3; ++t) {
-        const uint8_t* bb_ = bbase;
-        asm volatile("" : "+s"(bb_));
+      for (; MASK == MASK_ADD && t < t_hi && c_nxt == 3; ++t) {
         v4i bias_w[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) bias_w[i] = load_global_v4i(bb_ + (boff + 128u * (uint32_t)t + 16u * i));
+        SAGE_LOAD_BIAS(t, bias_w);
         const int tn_ = min(t + 1, t_hi - 1);
         c_nxt = mcls[tn_];
         SAGE_ISSUE_TILE(tn_, (t + 1) & 1);
@@ -820,6 +865,7 @@ __global__ __launch_bounds__(ATT_THREADS, attn_occupancy<layout_dim(HD)>()) void
     }
   }
 #undef SAGE_ISSUE_TILE
+#undef SAGE_LOAD_BIAS
 #undef SAGE_TILE
 #undef SAGE_TILE_PASSES
 
@@ -1125,7 +1171,7 @@ static int launch_attn(const int8_t* q8, const float* qs, const int8_t* k8, cons
   float* part = static_cast<float*>(workspace);
   hipLaunchKernelGGL((attn_kernel<HD, CAUSAL, OUT_DT, false>), dim3(blocks), dim3(ATT_THREADS), 0, st, q8, qs, k8, ks, v8t,
                      vs, o, osb, oss, osh, lse, H, Hkv, Sq, Skv, kv_pad(Skv), q_tiles, p.n_tiles, p.n_full, p.chunks,
-                     (int)p.p32, part, c0, hd, VarlenTiles{}, MaskTabs{}, nullptr, nullptr, nullptr, nullptr);
+                     (int)p.p32, part, c0, hd, VarlenTiles{}, MaskTabs{}, nullptr, nullptr, nullptr);
   if (n_split > 0) {
     if ((rc = check_launch("attention launch"))) return rc;
     launch_merge<D, OUT_DT>(p, n_split, part, qs, vs, o, osb, oss, osh, lse, H, Hkv, Sq, q_tiles, CAUSAL, c0, hd, st);
@@ -1203,7 +1249,7 @@ static int launch_attn_varlen(const int8_t* q8, const float* qs, const int8_t* k
   hipLaunchKernelGGL((attn_kernel<HD, CAUSAL, OUT_DT, true>), dim3(n_blocks), dim3(ATT_THREADS), 0, st, q8, qs, k8, ks,
                      v8t, vs, static_cast<uint16_t*>(out), (int64_t)0, oss, osh, nullptr, H, Hkv, TQ, 0, TKP, 0,
                      n_blocks, n_blocks, 1, 0, nullptr, logit_scale_base(hd), hd, vt, MaskTabs{}, nullptr, nullptr,
-                     nullptr, nullptr);
+                     nullptr);
   return check_launch("varlen attention launch");
 }
 
@@ -1233,7 +1279,7 @@ int attn_mask_plan_impl(int B, int H, int Sq, int Skv, int D, int64_t* ws) {
   return SAGE_OK;
 }
 
-template <int HD, bool CAUSAL, int OUT_DT>
+template <int HD, bool ADDITIVE, int OUT_DT>
 static int launch_attn_mask(const int8_t* q8, const float* qs, const int8_t* k8, const float* ks, const uint8_t* v8t,
                             const float* vs, void* out, int64_t osb, int64_t oss, int64_t osh, int B, int H, int Hkv,
                             int Sq, int Skv, int hd, MaskTabs mt, void* workspace, hipStream_t st) {
@@ -1247,9 +1293,10 @@ static int launch_attn_mask(const int8_t* q8, const float* qs, const int8_t* k8,
   const float c0 = logit_scale_base(hd);
   uint16_t* o = static_cast<uint16_t*>(out);
   float* part = static_cast<float*>(workspace);
-  hipLaunchKernelGGL((attn_kernel<HD, false, OUT_DT, false, true>), dim3(blocks), dim3(ATT_THREADS), 0, st, q8, qs, k8,
-                     ks, v8t, vs, o, osb, oss, osh, nullptr, H, Hkv, Sq, Skv, kv_pad(Skv), q_tiles, p.n_tiles,
-                     p.n_full, p.chunks, (int)p.p32, part, c0, hd, VarlenTiles{}, mt, mt.bits, mt.cls, mt.range, mt.bias);
+  hipLaunchKernelGGL((attn_kernel<HD, false, OUT_DT, false, ADDITIVE ? MASK_ADD : MASK_BOOL>), dim3(blocks),
+                     dim3(ATT_THREADS), 0, st, q8, qs, k8, ks, v8t, vs, o, osb, oss, osh, nullptr, H, Hkv, Sq, Skv,
+                     kv_pad(Skv), q_tiles, p.n_tiles, p.n_full, p.chunks, (int)p.p32, part, c0, hd, VarlenTiles{}, mt,
+                     mt.bits, mt.cls, mt.range);
   if (n_split > 0) {
     if ((rc = check_launch("masked attention launch"))) return rc;
     launch_merge<D, OUT_DT>(p, n_split, part, qs, vs, o, osb, oss, osh, nullptr, H, Hkv, Sq, q_tiles, 0, c0, hd, st);
@@ -1261,7 +1308,7 @@ static int launch_attn_mask(const int8_t* q8, const float* qs, const int8_t* k8,
 int attn_mask_impl(const int8_t* q8, const float* qs, const int8_t* k8, const float* ks, const uint8_t* v8t,
                    const float* vs, void* out, int64_t osb, int64_t oss, int64_t osh, int B, int H, int Hkv, int Sq,
                    int Skv, int D, int out_dtype, const MaskTabs* mt, void* workspace, void* stream) {
-  return SAGE_ATTN_DISPATCH(D, false, out_dtype == SAGE_DTYPE_BF16, launch_attn_mask, q8, qs, k8, ks, v8t, vs, out,
+  return SAGE_ATTN_DISPATCH(D, mt->raw != nullptr, out_dtype == SAGE_DTYPE_BF16, launch_attn_mask, q8, qs, k8, ks, v8t, vs, out,
                             osb, oss, osh, B, H, Hkv, Sq, Skv, D, *mt, workspace, (hipStream_t)stream);
 }
 

@@ -48,6 +48,13 @@ template <int DT> __device__ __forceinline__ uint32_t f32_to_out_bits(float f) {
   return DT == DT_BF16 ? f32_to_bf16_bits(f) : f32_to_f16_bits(f);
 }
 
+// 16 bytes of 16-bit elements at an address aligned to one element
+typedef uint32_t v4u_a2 __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ v4i load16_2aligned(const void* p) {
+  const v4u_a2 w = *(const __attribute__((address_space(1))) v4u_a2*)(p);
+  return v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+}
+
 // ---- cross-lane moves -------------------------------------------------------------------------------------------
 // DPP quad_perm selectors: lane i of each quad reads lane sel[i].
 constexpr int DPP_QUAD_XOR1 = 0xB1;  // [1, 0, 3, 2]

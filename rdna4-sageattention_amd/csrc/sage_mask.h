@@ -16,24 +16,60 @@ struct MaskPrep {
   int64_t msb, msh, msq;
   int mh, mq, mg, nt, nrb;  // table extents (sage_mask.hip: mask_shape)
   int Sq, Skv, causal;
-  int a4;                   // mask rows aligned to a run of 4 keys (4 bytes bool, 8 bytes 16-bit): one load per run
+  int a4;                   // bool rows aligned to a run of 4 keys (4 bytes): one load per run
   uint32_t* bits;
-  uint16_t* bias;           // 16-bit masks: the values of class-3 tiles, 32 per (row, tile, lane half), lane order
+  uint16_t* bias;           // 16-bit masks: the 64 values of every row's partial last tile (-inf past kv_len)
   int* cls;
   int2* range;
   int nrange;               // mb * mh * nrb
   int prep_blocks, range_blocks;
 };
 
+typedef unsigned short v2us __attribute__((ext_vector_type(2)));
+
+// 1 in each 16-bit half of x that is not 0
+__device__ __forceinline__ uint32_t nonzero_halves(uint32_t x) {
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(v2us, x), v2us{1, 1}));
+}
+
+// The visibility word of the lane's 32 keys of a bool mask (bit order below); keys past `lim` are not visible.
+__device__ __forceinline__ uint32_t mask_bool_word(const MaskPrep& p, const uint8_t* row, int k0, int lim) {
+  uint32_t b4[8], w = 0;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int kj = k0 + 8 * j;
+    if (p.a4 && kj + 3 < p.Skv) {
+      b4[j] = *reinterpret_cast<const uint32_t*>(row + kj);
+    } else {
+      b4[j] = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (kj + i < p.Skv) b4[j] |= (uint32_t)row[kj + i] << (8 * i);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const bool vis = ((b4[j] >> (8 * i)) & 0xFFu) != 0 && k0 + 8 * j + i <= lim;
+      w |= (uint32_t)vis << (4 * j + i);
+    }
+  return w;
+}
+
 // One wave per (mask batch-head, 32-row group, tile); a block is 4 waves on 4 consecutive tiles.  Lane (row r =
-// lane % 32 of the group, half hf = lane / 32) reads the 32 mask elements of its keys (8 runs of 4 consecutive keys:
-// run j holds keys 64 t + 8 j + 4 hf + i at bits 4 j + i, values 4 j + i of the lane's bias entry).  Bool masks:
-// a key is visible when its byte is nonzero.  16-bit (additive) masks: when its value is not -inf; the lane's keys
-// are also "zero" (every value +-0) or "general" (some value neither 0 nor -inf).  Keys past kv_len and, causal,
-// past the bottom-right diagonal are -inf.  Wave ballots give the class: 0 no row sees a key, 1 every key of every
-// row visible with a zero bias, 2 visibility only (bool masks, or 16-bit values all 0 / -inf), 3 a general bias, whose
-// values each lane then stores (-inf where masked).  Rows past q_len (and, for a mask without rows, every row but 0)
+// lane % 32 of the group, half hf = lane / 32) writes the visibility word of its 32 keys: bits 4 j + i for key
+// 64 t + 8 j + 4 hf + i.  Bool masks: the lane reads those keys (8 runs of 4); a key is visible when its byte is
+// nonzero.  16-bit (additive) masks: the two lanes of a row read alternate 16-byte chunks (8 keys each) and exchange
+// the half-words the other one needs; a key is visible when its value is not -inf; the values a lane reads are also
+// "zero" (every one +-0) or "general" (some value neither 0 nor -inf).  Keys past kv_len and, causal, past the
+// bottom-right diagonal are -inf.  Wave ballots give the class: 0 no row sees a key, 1 every key of every row visible
+// with a zero bias, 2 visibility only (bool masks, or 16-bit values all 0 / -inf), 3 a general bias.  The attention
+// reads the values of class-3 tiles from the mask itself; only those of a partial last tile are copied here, padded
+// with -inf, so that it never reads past a row's end.  Rows past q_len (and, for a mask without rows, every row but 0)
 // count as neither seeing nor missing a key.  block < mb * mh * mg * ceil(nt / 4).
+//
+// A 16-bit mask is read once here (HBM bound) and once by the attention.
 __device__ __forceinline__ void mask_prep_block(const MaskPrep& p, int block) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int r = lane & 31, hf = lane >> 5;
@@ -46,76 +82,78 @@ __device__ __forceinline__ void mask_prep_block(const MaskPrep& p, int block) {
   const int mbi = mbh / p.mh, mhi = mbh % p.mh;
   const int q = g * 32 + r;  // table row (mq == 1: row 0 only)
   const bool real = p.mq == 1 ? r == 0 : q < p.Sq;
-  const int64_t entry = ((int64_t)mbh * p.mq + q) * p.nt + t;  // (row, tile) of the tables
   uint32_t w = 0;
   bool zero = true, general = false;
-  uint32_t vals[16];  // 16-bit masks: the lane's 32 values, two per word, -inf where masked
+  v4i c[4] = {};  // 16-bit masks: the lane's chunks, keys [64 t + 16 i + 8 hf, + 8)
+  const bool part = (t + 1) * 64 > p.Skv;
   if (real) {
     const int lim = p.causal ? min(p.Skv - 1, q + (p.Skv - p.Sq)) : p.Skv - 1;  // last key the row may see
-    const int k0 = t * 64 + 4 * hf;
     const int64_t rowoff = mbi * p.msb + mhi * p.msh + (int64_t)q * p.msq;
     if (p.mdt == SAGE_DTYPE_BOOL) {
-      const uint8_t* row = static_cast<const uint8_t*>(p.mask) + rowoff;
-      uint32_t b4[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int kj = k0 + 8 * j;
-        if (p.a4 && kj + 3 < p.Skv) {
-          b4[j] = *reinterpret_cast<const uint32_t*>(row + kj);
-        } else {
-          b4[j] = 0;
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (kj + i < p.Skv) b4[j] |= (uint32_t)row[kj + i] << (8 * i);
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const bool vis = ((b4[j] >> (8 * i)) & 0xFFu) != 0 && k0 + 8 * j + i <= lim;
-          w |= (uint32_t)vis << (4 * j + i);
-        }
+      w = mask_bool_word(p, static_cast<const uint8_t*>(p.mask) + rowoff, t * 64 + 4 * hf, lim);
     } else {
-      const uint16_t* row = static_cast<const uint16_t*>(p.mask) + rowoff;
-      const uint16_t ninf = p.mdt == SAGE_DTYPE_BF16 ? 0xFF80u : 0xFC00u;
+      const uint32_t ninf = p.mdt == SAGE_DTYPE_BF16 ? 0xFF80u : 0xFC00u;
+      const uint16_t* row = static_cast<const uint16_t*>(p.mask) + rowoff + t * 64 + 8 * hf;
+      const int left = lim - t * 64 - 8 * hf;  // the lane's key 16 i + e is visible when 16 i + e <= left
+      if (!part) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int kj = k0 + 8 * j;
-        uint16_t e[4];
-        if (p.a4 && kj + 3 < p.Skv) {
-          const uint2 u = *reinterpret_cast<const uint2*>(row + kj);
-          e[0] = (uint16_t)(u.x & 0xFFFFu);
-          e[1] = (uint16_t)(u.x >> 16);
-          e[2] = (uint16_t)(u.y & 0xFFFFu);
-          e[3] = (uint16_t)(u.y >> 16);
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) e[i] = kj + i < p.Skv ? row[kj + i] : ninf;
-        }
+        for (int i = 0; i < 4; ++i) c[i] = load16_2aligned(row + 16 * i);
+      } else {
+        const int in_row = p.Skv - 1 - t * 64 - 8 * hf;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          if (k0 + 8 * j + i > lim) e[i] = ninf;
-          const bool vis = e[i] != ninf;
-          const bool z = (e[i] & 0x7FFFu) == 0;
-          w |= (uint32_t)vis << (4 * j + i);
-          zero = zero && z;
-          general = general || (vis && !z);
+          uint32_t e[8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) e[u] = 16 * i + u <= in_row ? (uint32_t)row[16 * i + u] : ninf;
+#pragma unroll
+          for (int d = 0; d < 4; ++d) c[i][d] = (int)(e[2 * d] | (e[2 * d + 1] << 16));
         }
-        vals[2 * j] = (uint32_t)e[0] | ((uint32_t)e[1] << 16);
-        vals[2 * j + 1] = (uint32_t)e[2] | ((uint32_t)e[3] << 16);
       }
+      if (p.causal && t * 64 + 63 > g * 32 + (p.Skv - p.Sq)) {  // wave-uniform: the tile crosses some row's diagonal
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+          for (int d = 0; d < 4; ++d) {
+            uint32_t x = (uint32_t)c[i][d];
+            if (16 * i + 2 * d > left) x = (x & 0xFFFF0000u) | ninf;
+            if (16 * i + 2 * d + 1 > left) x = (x & 0xFFFFu) | (ninf << 16);
+            c[i][d] = (int)x;
+          }
+        }
+      }
+      uint32_t anynz = 0, gen = 0, lo = 0, hi = 0;  // lo / hi: visibility of the chunks' first / last 4 keys
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          const uint32_t nz = nonzero_halves((uint32_t)c[i][d] & 0x7FFF7FFFu);
+          const uint32_t vis = nonzero_halves((uint32_t)c[i][d] ^ (ninf * 0x10001u));
+          anynz |= nz;
+          gen |= nz & vis;
+          const uint32_t two = (vis | (vis >> 15)) & 3u;
+          if (d < 2)
+            lo |= two << (8 * i + 2 * d);
+          else
+            hi |= two << (8 * i + 2 * (d - 2));
+        }
+      }
+      zero = anynz == 0;
+      general = gen != 0;
+      // lane hf holds the chunks j = 2 i + hf (bits 4 j): its own half of them is the word's, the other half goes to
+      // the row's other lane
+      const auto x = __builtin_amdgcn_permlane32_swap(lo << (4 * hf), hi << (4 * hf), false, false);
+      w = x[0] | x[1];
     }
-    p.bits[entry * 2 + hf] = w;
+    p.bits[((int64_t)mbh * p.mq + q) * p.nt * 2 + t * 2 + hf] = w;
   }
   const uint64_t any = __ballot(real && w != 0);
   const uint64_t all = __ballot(!real || (w == 0xFFFFFFFFu && zero));
   const uint64_t gen = __ballot(real && general);
   const int cls = any == 0 ? 0 : gen != 0 ? 3 : all == ~0ull ? 1 : 2;
-  if (cls == 3 && real) {  // wave-uniform class
-    uint4* dst = reinterpret_cast<uint4*>(p.bias + (entry * 2 + hf) * 32);
+  if (cls == 3 && part && real) {  // wave-uniform class
+    uint16_t* dst = p.bias + ((int64_t)mbh * p.mq + q) * 64 + 8 * hf;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) dst[i] = make_uint4(vals[4 * i], vals[4 * i + 1], vals[4 * i + 2], vals[4 * i + 3]);
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<v4i*>(dst + 16 * i) = c[i];
   }
   if (lane == 0) p.cls[((int64_t)mbh * p.mg + g) * p.nt + t] = cls;
 }

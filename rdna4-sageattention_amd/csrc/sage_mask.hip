@@ -9,7 +9,8 @@
 //   cls   one entry per (32-row group, tile): 0 = no row sees a key of the tile (the wave skips it), 1 = every row
 //         sees every key with a zero bias (the mask-free tile body), 2 = mixed visibility (the bit-masked body),
 //         3 = an additive bias (float masks only: the biased body);
-//   bias  float masks: the 16-bit values of class-3 tiles in the bits' lane order, 32 per word;
+//   bias  float masks: the 64 16-bit values of every row's last tile when kv_len is not a multiple of 64 (-inf past
+//         it); the other class-3 tiles are read from the mask itself;
 //   range one (first, last + 1) tile pair per 128-row block (an attention workgroup's rows): the tiles outside it
 //         are not visited at all.
 // Keys past kv_len and, with the causal flag, keys past the bottom-right diagonal are folded into the bits.  The
@@ -56,7 +57,7 @@ static MaskShape mask_shape(int B, int H, int Sq, int Skv, int64_t msb, int64_t 
 static int64_t align256(int64_t n) { return (n + 255) / 256 * 256; }
 
 // Workspace of sage_forward_masked: the attention plan's split state, the per-chunk V maxima, the bits, the classes,
-// the ranges, and for a float mask the bias values (each 256-byte aligned).
+// the ranges, and for a float mask the rows' partial last tiles (each 256-byte aligned).
 struct MaskWorkspace {
   int64_t attn, vpart, bits, cls, range, bias, total;
 };
@@ -69,7 +70,7 @@ static int mask_workspace(int B, int H, int Hkv, int Sq, int Skv, int D, const M
   w->cls = w->bits + align256(m.bits_words * 4);
   w->range = w->cls + align256(m.cls_entries * 4);
   w->bias = w->range + align256(m.range_entries * 8);
-  w->total = w->bias + (m.additive ? align256(m.bits_words * 32 * 2) : 0);
+  w->total = w->bias + (m.additive && Skv % 64 ? align256((int64_t)m.mb * m.mh * m.mq * 64 * 2) : 0);
   return SAGE_OK;
 }
 
@@ -84,7 +85,8 @@ static int check_mask_shape(int B, int H, int Hkv, int Sq, int Skv, int D, int c
   if (mask_dtype != SAGE_DTYPE_BOOL && mask_dtype != SAGE_DTYPE_BF16 && mask_dtype != SAGE_DTYPE_F16)
     return fail(SAGE_ERR_UNSUPPORTED, "%s: mask dtype code %d (bool=2, bf16=0, f16=1)", who, mask_dtype);
   const MaskShape m = mask_shape(B, H, Sq, Skv, msb, msh, msq, causal, mask_dtype);
-  // the kernel addresses one (batch, head) slice of the bits (and of the bias values: 16x) with a 32-bit byte offset
+  // the kernel addresses one (batch, head) slice of the bits with a 32-bit byte offset (additive masks: the bound of
+  // a table of their values)
   SAGE_REQUIRE((int64_t)m.mq * m.nt * (m.additive ? 128 : 8) < (1ll << 31), "%s: mask of %d rows x %d keys too large",
                who, Sq, Skv);
   SAGE_REQUIRE(m.cls_entries < (1ll << 31) && (int64_t)B * H * ((Sq + 127) / 128) * 16 < (1ll << 31),
@@ -158,11 +160,10 @@ int sage_forward_masked(const void* q, int64_t qsb, int64_t qss, int64_t qsh, co
   mp.Sq = Sq;
   mp.Skv = Skv;
   mp.causal = causal;
-  // a run of 4 keys as one load: 4 bytes (bool) or 8 bytes (16-bit) aligned rows
-  const unsigned run_bytes = mask_dtype == SAGE_DTYPE_BOOL ? 4u : 8u;
-  mp.a4 = ((uintptr_t)mask % run_bytes) == 0 && msb % 4 == 0 && msh % 4 == 0 && msq % 4 == 0;
+  // bool: a run of 4 keys as one load where the rows are 4-byte aligned
+  mp.a4 = ((uintptr_t)mask % 4) == 0 && msb % 4 == 0 && msh % 4 == 0 && msq % 4 == 0;
   mp.bits = bits;
-  mp.bias = m.additive ? reinterpret_cast<uint16_t*>(ws + w.bias) : nullptr;
+  mp.bias = m.additive && Skv % 64 ? reinterpret_cast<uint16_t*>(ws + w.bias) : nullptr;
   mp.cls = cls;
   mp.range = range;
   mp.nrange = (int)m.range_entries;
@@ -174,6 +175,7 @@ int sage_forward_masked(const void* q, int64_t qsb, int64_t qss, int64_t qsh, co
   const sage::MaskTabs mt{bits,
                           cls,
                           range,
+                          m.additive ? static_cast<const uint16_t*>(mask) : nullptr,
                           mp.bias,
                           m.mb > 1 ? (int64_t)m.mh * m.mq * m.nt * 2 : 0,
                           m.mh > 1 ? (int64_t)m.mq * m.nt * 2 : 0,
@@ -183,6 +185,13 @@ int sage_forward_masked(const void* q, int64_t qsb, int64_t qss, int64_t qsh, co
                           m.mg > 1 ? (int64_t)m.nt : 0,
                           m.mb > 1 ? (int64_t)m.mh * m.nrb : 0,
                           m.mh > 1 ? (int64_t)m.nrb : 0,
+                          msb,
+                          msh,
+                          msq,
+                          m.mb > 1 ? (int64_t)m.mh * m.mq * 64 : 0,
+                          m.mh > 1 ? (int64_t)m.mq * 64 : 0,
+                          m.mq > 1 ? (int64_t)64 : 0,
+                          causal,
                           m.mg,
                           m.nrb};
   return sage::attn_mask_impl(q8, qs, k8, ks, v8t, vs, out, osb, oss, osh, B, H, Hkv, Sq, Skv, D, dtype, &mt,
