@@ -142,12 +142,17 @@ struct VarlenTiles {
 // (classes 0-2) or MASK_ADD (additive, class 3 as well; apart because its tile body costs the other bodies registers).
 constexpr int MASK_NONE = 0, MASK_BOOL = 1, MASK_ADD = 2;
 constexpr int64_t MASK_ROW_32BIT = 1 << 26;  // 31 rows of at most this many 16-bit elements: a 32-bit byte offset
-template <int HD, bool CAUSAL, int OUT_DT, bool VARLEN, int MASK = MASK_NONE>
+// PART: the format of a split tile's partials, fp16 or fp32, or (mask variants) by the argument p32.  Two kernels rather
+// than two epilogues in one: with both, the fp16 launches lost 1.4% (Flux, 158.1 -> 160.4 us; 13.8 -> 14.2 us at
+// 1x8x1024x64).
+constexpr int PART_F16 = 0, PART_F32 = 1, PART_ANY = 2;
+constexpr int part_format(bool causal, int mask) { return mask ? PART_ANY : causal ? PART_F32 : PART_F16; }
+template <int HD, bool CAUSAL, int OUT_DT, bool VARLEN, int MASK = MASK_NONE, int PART = part_format(CAUSAL, MASK)>
 __global__ __launch_bounds__(ATT_THREADS, (attn_occupancy<layout_dim(HD), MASK == MASK_ADD>())) void attn_kernel(
     const int8_t* __restrict__ q8, const float* __restrict__ qs, const int8_t* __restrict__ k8,
     const float* __restrict__ ks, const uint8_t* __restrict__ v8t, const float* __restrict__ vs,
     uint16_t* __restrict__ out, int64_t osb, int64_t oss, int64_t osh, float* __restrict__ lse, int H, int Hkv,
-    int Sq_arg, int Skv_arg, int Skp, int q_tiles, int total, int n_full, int chunks, int p32, float* __restrict__ part,
+    int Sq_arg, int Skv_arg, int Skp, int q_tiles, int total, int n_full, int chunks, int p32_arg, float* __restrict__ part,
     float c0, int dout, VarlenTiles vt, MaskTabs mt, const uint32_t* __restrict__ mbits_tab,
     const int* __restrict__ mcls_tab, const int2* __restrict__ mrange_tab) {
   static_assert(!(MASK && (CAUSAL || VARLEN)), "the mask variant folds causality into its bits and is dense only");
@@ -181,6 +186,7 @@ __global__ __launch_bounds__(ATT_THREADS, (attn_occupancy<layout_dim(HD), MASK =
   // for one workgroup per CU) and for the mask variant (whose loops prefetch one tile ahead)
   constexpr int NBUF = (!MASK && D <= 128) ? 3 : 2;
   constexpr int LPT = KLOADS + VLOADS;  // direct loads per wave and tile
+  const bool p32 = PART == PART_ANY ? p32_arg != 0 : PART == PART_F32;
   __shared__ __attribute__((aligned(16))) uint8_t smem[NBUF][TILE];
 
   // ---- work decode.  Dense: blocks [0, n_full) own whole query tiles (XCD-grouped; causal: longest first); each
@@ -904,7 +910,7 @@ __global__ __launch_bounds__(ATT_THREADS, (attn_occupancy<layout_dim(HD), MASK =
     }
     const int64_t units = (int64_t)(total - n_full) * chunks;
     if (hf == 0)
-      reinterpret_cast<float2*>(reinterpret_cast<uint8_t*>(part) + ws_ml_offset(units, D, p32 != 0))[(int64_t)unit * ATT_BM + q] =
+      reinterpret_cast<float2*>(reinterpret_cast<uint8_t*>(part) + ws_ml_offset(units, D, p32))[(int64_t)unit * ATT_BM + q] =
           make_float2(m * SSCALE, lt);  // m in S * ks units, as the merge kernel's cl expects
     return;
   }
@@ -947,21 +953,19 @@ __global__ __launch_bounds__(ATT_THREADS, (attn_occupancy<layout_dim(HD), MASK =
 // O = sum_i W_i * (O_i / l_i) as stored, fp32 with P32 and fp16 otherwise (float32, chunk order), the output is (O * ((1/448) / L)) * VS and
 // lse = ln2 * (cl * M + log2 L), the epilogue of an unsplit tile.  grid = n_split * 128 * (D / 4) / 256 blocks of 256 threads.
 // ------------------------------------------------------------------------------------------------------------------
-template <int D, int OUT_DT, bool P32>
+template <int D, int OUT_DT, bool P32, bool CAUSAL>
 __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict__ part, const float* __restrict__ qs,
                                                          const float* __restrict__ vs, uint16_t* __restrict__ out,
                                                          int64_t osb, int64_t oss, int64_t osh,
                                                          float* __restrict__ lse, int H, int Hkv, int Sq, int q_tiles,
-                                                         int n_full, int n_split, int chunks, int causal, float c0,
-                                                         int dout) {
-  constexpr int NG = D / 4;
-  const int idx = blockIdx.x * 256 + threadIdx.x;
-  const int cg = idx % NG;
+                                                         int n_full, int n_split, int chunks, float c0, int dout) {
+  constexpr int NG = D / 4, ROWS = 256 / NG, BPT = ATT_BM / ROWS;  // rows per block, blocks per tile
+  const int cg = threadIdx.x % NG;
   if (4 * cg >= dout) return;  // head_dim 96: padding channels
-  const int q = (idx / NG) % ATT_BM;
-  const int s = idx / (NG * ATT_BM);
+  const int s = blockIdx.x / BPT;  // a block lies inside one tile, so the tile's indexes are scalar
+  const int q = blockIdx.x % BPT * ROWS + threadIdx.x / NG;
   int bh = (n_full + s) / q_tiles, qt = (n_full + s) % q_tiles;
-  if (causal) causal_tile(n_full + s, (n_full + n_split) / q_tiles, q_tiles, bh, qt);
+  if (CAUSAL) causal_tile(n_full + s, (n_full + n_split) / q_tiles, q_tiles, bh, qt);
   const int qrow = qt * ATT_BM + q;
   if (qrow >= Sq) return;
   const int b = bh / H, h = bh % H;
@@ -1129,17 +1133,15 @@ static int make_plan(int B, int H, int Sq, int Skv, AttnPlan* p) {
 // c0 = log2(e) / sqrt(head_dim) with the kernel's built-in sm_scale (other scales are folded into QS)
 static float logit_scale_base(int head_dim) { return (float)((1.0 / __builtin_sqrt((double)head_dim)) * 1.4426950408889634); }
 
-template <int D, int OUT_DT>
+template <int D, int OUT_DT, bool CAUSAL>
 static void launch_merge(const AttnPlan& p, int n_split, const float* part, const float* qs, const float* vs,
                          uint16_t* out, int64_t osb, int64_t oss, int64_t osh, float* lse, int H, int Hkv, int Sq,
-                         int q_tiles, int causal, float c0, int hd, hipStream_t st) {
-  const dim3 grid(n_split * (ATT_BM * D / 4 / 256));
-  if (p.p32)
-    hipLaunchKernelGGL((attn_merge_kernel<D, OUT_DT, true>), grid, dim3(256), 0, st, part, qs, vs, out, osb, oss, osh,
-                       lse, H, Hkv, Sq, q_tiles, p.n_full, n_split, p.chunks, causal, c0, hd);
-  else
-    hipLaunchKernelGGL((attn_merge_kernel<D, OUT_DT, false>), grid, dim3(256), 0, st, part, qs, vs, out, osb, oss, osh,
-                       lse, H, Hkv, Sq, q_tiles, p.n_full, n_split, p.chunks, causal, c0, hd);
+                         int q_tiles, float c0, int hd, hipStream_t st) {
+  auto* kernel = attn_merge_kernel<D, OUT_DT, true, CAUSAL>;
+  if constexpr (!CAUSAL)
+    if (!p.p32) kernel = attn_merge_kernel<D, OUT_DT, false, false>;
+  hipLaunchKernelGGL(kernel, dim3(n_split * (ATT_BM * D / 4 / 256)), dim3(256), 0, st, part, qs, vs, out, osb, oss, osh, lse,
+                     H, Hkv, Sq, q_tiles, p.n_full, n_split, p.chunks, c0, hd);
 }
 
 // HD: head dim (64, 96, 128, 256); D = layout_dim(HD) channels of the intermediates (96 runs on the 128-channel
@@ -1169,12 +1171,15 @@ static int launch_attn(const int8_t* q8, const float* qs, const int8_t* k8, cons
   const float c0 = logit_scale_base(hd);
   uint16_t* o = static_cast<uint16_t*>(out);
   float* part = static_cast<float*>(workspace);
-  hipLaunchKernelGGL((attn_kernel<HD, CAUSAL, OUT_DT, false>), dim3(blocks), dim3(ATT_THREADS), 0, st, q8, qs, k8, ks, v8t,
-                     vs, o, osb, oss, osh, lse, H, Hkv, Sq, Skv, kv_pad(Skv), q_tiles, p.n_tiles, p.n_full, p.chunks,
-                     (int)p.p32, part, c0, hd, VarlenTiles{}, MaskTabs{}, nullptr, nullptr, nullptr);
+  auto* kernel = attn_kernel<HD, CAUSAL, OUT_DT, false>;
+  if constexpr (!CAUSAL)
+    if (p.p32) kernel = attn_kernel<HD, false, OUT_DT, false, MASK_NONE, PART_F32>;
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(ATT_THREADS), 0, st, q8, qs, k8, ks, v8t, vs, o, osb, oss, osh, lse, H, Hkv,
+                     Sq, Skv, kv_pad(Skv), q_tiles, p.n_tiles, p.n_full, p.chunks, (int)p.p32, part, c0, hd, VarlenTiles{},
+                     MaskTabs{}, nullptr, nullptr, nullptr);
   if (n_split > 0) {
     if ((rc = check_launch("attention launch"))) return rc;
-    launch_merge<D, OUT_DT>(p, n_split, part, qs, vs, o, osb, oss, osh, lse, H, Hkv, Sq, q_tiles, CAUSAL, c0, hd, st);
+    launch_merge<D, OUT_DT, CAUSAL>(p, n_split, part, qs, vs, o, osb, oss, osh, lse, H, Hkv, Sq, q_tiles, c0, hd, st);
   }
   return check_launch("attention launch");
 }
@@ -1299,7 +1304,7 @@ static int launch_attn_mask(const int8_t* q8, const float* qs, const int8_t* k8,
                      mt.bits, mt.cls, mt.range);
   if (n_split > 0) {
     if ((rc = check_launch("masked attention launch"))) return rc;
-    launch_merge<D, OUT_DT>(p, n_split, part, qs, vs, o, osb, oss, osh, nullptr, H, Hkv, Sq, q_tiles, 0, c0, hd, st);
+    launch_merge<D, OUT_DT, false>(p, n_split, part, qs, vs, o, osb, oss, osh, nullptr, H, Hkv, Sq, q_tiles, c0, hd, st);
   }
   return check_launch("masked attention launch");
 }
