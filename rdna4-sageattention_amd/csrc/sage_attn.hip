@@ -898,13 +898,17 @@ __global__ __launch_bounds__(ATT_THREADS, (attn_occupancy<layout_dim(HD), MASK =
         }
     } else {
       uint16_t* po = reinterpret_cast<uint16_t*>(part) + ((int64_t)unit * ATT_BM + q) * D;
+      // the product and its fp16 rounding are one v_fma_mixlo_f16 (one rounding); a product shared with the fp32 branch
+      // above would be rounded twice, and the mask variants would differ from the unmasked kernel in a few last bits
+      float rl16 = rl;
+      asm volatile("" : "+v"(rl16));
 #pragma unroll
       for (int i = 0; i < NPV; ++i)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           uint32_t e[4];
 #pragma unroll
-          for (int u = 0; u < 4; ++u) e[u] = f32_to_f16_bits((o[i][4 * g + u] * ls) * rl);
+          for (int u = 0; u < 4; ++u) e[u] = f32_to_f16_bits((o[i][4 * g + u] * ls) * rl16);
           *reinterpret_cast<uint2*>(po + 32 * i + 8 * g + 4 * hf) = make_uint2(e[0] | (e[1] << 16), e[2] | (e[3] << 16));
         }
     }

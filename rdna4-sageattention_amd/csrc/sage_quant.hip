@@ -7,6 +7,7 @@
 //  quant_kv_kernel  K rows -> Hadamard -> int8, one scale per 32 keys; V -> E4M3 with the per-channel scale,
 //                   transposed through LDS into V8T                                  (sage_quant.py:51-70)
 //  quant_qk_vamax_kernel, quant_v_kernel   the same work in sage_forward's two launches
+//  quant_short_kernel   the same work in one launch, for short key ranges
 //  quant_varlen_kernel, quant_v_varlen_kernel   packed variable-length batches
 //
 // Row mapping of the Hadamard kernels: 4 lanes (one quad) per row, each lane owns DP / 4 consecutive elements
@@ -257,6 +258,52 @@ __device__ __forceinline__ void quant_k_rows64(const uint16_t* __restrict__ k, i
                         ks + (int64_t)bh * (Skp / SAGE_KV_BLOCK) + blk * 2);
 }
 
+// 8 channels of one V row (16 bytes) times their scales cs = 448 / max, as E4M3 in two words.  The hardware conversion
+// rounds to nearest even with subnormals; its inputs are within +-448.
+template <int DT>
+__device__ __forceinline__ void v_to_e4m3(const uint4& x, const float (&cs)[8], uint32_t& t0, uint32_t& t1) {
+  const uint32_t ws[4] = {x.x, x.y, x.z, x.w};
+  float y[8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    y[2 * i] = fminf(fmaxf(elem_lo<DT>(ws[i]) * cs[2 * i], -448.0f), 448.0f);
+    y[2 * i + 1] = fminf(fmaxf(elem_hi<DT>(ws[i]) * cs[2 * i + 1], -448.0f), 448.0f);
+  }
+  int a = __builtin_amdgcn_cvt_pk_fp8_f32(y[0], y[1], 0, false);
+  a = __builtin_amdgcn_cvt_pk_fp8_f32(y[2], y[3], a, true);
+  int b = __builtin_amdgcn_cvt_pk_fp8_f32(y[4], y[5], 0, false);
+  b = __builtin_amdgcn_cvt_pk_fp8_f32(y[6], y[7], b, true);
+  t0 = (uint32_t)a;
+  t1 = (uint32_t)b;
+}
+
+// Transposed store of an LDS tile [keys][channels] of E4M3 bytes with row pitch PITCH: 16 output positions of 4
+// channels.  Key set ksel = 4G + u covers the positions [64G + 16u, +16), i.e. keys 64G + 8g + 4h + r with h = u / 2,
+// g = 4(u % 2) + i.  `dst` = channel 4 cg at the tile's first position, channels chan_stride apart.
+template <int PITCH>
+__device__ __forceinline__ void v_store_set(const uint8_t* tile, int ksel, int cg, uint8_t* __restrict__ dst,
+                                            int64_t chan_stride) {
+  const int G = ksel >> 2, u = ksel & 3, hh = u >> 1;
+  uint32_t wd[4][4];  // [chunk i][key r] -> 4 channel bytes
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int g = 4 * (u & 1) + i;
+#pragma unroll
+    for (int rk = 0; rk < 4; ++rk)
+      wd[i][rk] = *reinterpret_cast<const uint32_t*>(tile + (64 * G + 8 * g + 4 * hh + rk) * PITCH + cg * 4);
+  }
+#pragma unroll
+  for (int ci = 0; ci < 4; ++ci) {
+    uint32_t o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      o[i] = ((wd[i][0] >> (8 * ci)) & 0xFFu) | (((wd[i][1] >> (8 * ci)) & 0xFFu) << 8) |
+             (((wd[i][2] >> (8 * ci)) & 0xFFu) << 16) | (((wd[i][3] >> (8 * ci)) & 0xFFu) << 24);
+    }
+    *reinterpret_cast<uint4*>(dst + (int64_t)ci * chan_stride + 64 * G + 16 * u) = make_uint4(o[0], o[1], o[2], o[3]);
+  }
+}
+
 // ------------------------------------------------------------------------------------------------------------------
 // V: E4M3 with the per-channel scale 448 / max(VS, 1e-30), 128 keys per block, transposed through LDS into V8T.
 // Core: local rows [local0, local0 + 128) of one (batch, kv head), `base` = row 0 of its source, rows >= nvalid are
@@ -340,51 +387,16 @@ __device__ __forceinline__ void quant_v128_core(const uint16_t* __restrict__ bas
 #pragma unroll
   for (int g = 0; g < 128 / RPI; ++g) {
     const int rr = r0 + g * RPI;
-    const uint32_t ws[4] = {wv[g].x, wv[g].y, wv[g].z, wv[g].w};
-    float y[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      y[2 * i] = fminf(fmaxf(elem_lo<DT>(ws[i]) * cs[2 * i], -448.0f), 448.0f);
-      y[2 * i + 1] = fminf(fmaxf(elem_hi<DT>(ws[i]) * cs[2 * i + 1], -448.0f), 448.0f);
-    }
-    // hardware E4M3 conversion (round to nearest even, subnormals kept; inputs are within +-448)
-    int t0 = __builtin_amdgcn_cvt_pk_fp8_f32(y[0], y[1], 0, false);
-    t0 = __builtin_amdgcn_cvt_pk_fp8_f32(y[2], y[3], t0, true);
-    int t1 = __builtin_amdgcn_cvt_pk_fp8_f32(y[4], y[5], 0, false);
-    t1 = __builtin_amdgcn_cvt_pk_fp8_f32(y[6], y[7], t1, true);
-    *reinterpret_cast<uint2*>(vtile + rr * PITCH + c8 * 8) = make_uint2((uint32_t)t0, (uint32_t)t1);
+    uint32_t t0, t1;
+    v_to_e4m3<DT>(wv[g], cs, t0, t1);
+    *reinterpret_cast<uint2*>(vtile + rr * PITCH + c8 * 8) = make_uint2(t0, t1);
   }
   __syncthreads();
 
-  // ---- V: transposed store.  Thread -> (4-channel group cg, 16-key set ksel); key set ksel = 4G + u covers output
-  // positions [64G + 16u, +16) of this 128-key block, i.e. keys 64G + 8g + 4h + r with h = u / 2, g = 4(u % 2) + i.
+  // ---- V: transposed store, a 4-channel group and 16 output positions per thread ----
   constexpr int NCG = DP / 4;
-  for (int item = threadIdx.x; item < NCG * 8; item += 256) {
-    const int ksel = item % 8, cg = item / 8;
-    const int G = ksel >> 2, u = ksel & 3, hh = u >> 1;
-    uint32_t wd[4][4];  // [chunk i][key r] -> 4 channel bytes
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int g = 4 * (u & 1) + i;
-#pragma unroll
-      for (int rk = 0; rk < 4; ++rk) {
-        const int key = 64 * G + 8 * g + 4 * hh + rk;
-        wd[i][rk] = *reinterpret_cast<const uint32_t*>(vtile + key * PITCH + cg * 4);
-      }
-    }
-#pragma unroll
-    for (int ci = 0; ci < 4; ++ci) {
-      uint32_t o[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        o[i] = ((wd[i][0] >> (8 * ci)) & 0xFFu) | (((wd[i][1] >> (8 * ci)) & 0xFFu) << 8) |
-               (((wd[i][2] >> (8 * ci)) & 0xFFu) << 16) | (((wd[i][3] >> (8 * ci)) & 0xFFu) << 24);
-      }
-      const int d = cg * 4 + ci;
-      uint8_t* dst = v8t_blk + (int64_t)d * chan_stride + 64 * G + 16 * u;
-      *reinterpret_cast<uint4*>(dst) = make_uint4(o[0], o[1], o[2], o[3]);
-    }
-  }
+  for (int item = threadIdx.x; item < NCG * 8; item += 256)
+    v_store_set<PITCH>(vtile, item % 8, item / 8, v8t_blk + (int64_t)(item / 8 * 4) * chan_stride, chan_stride);
 }
 
 // dense layout: grid = (Skp / 128) * B * Hkv blocks; vs_out (vchunks > 0) is written by block 0 of each (b, kv head)
@@ -403,13 +415,126 @@ __device__ __forceinline__ void quant_v_rows(const uint16_t* __restrict__ v, int
                          v8t + (int64_t)bh * DP * Skp + blk * 128, Skp);
 }
 
-// sage_forward's first launch: blocks [0, nv) write per-chunk V maxima (vamax_chunk_rows keys each) to `vpart`,
-// blocks [nv, nv + nk) quantize 64 keys of K each, the next nq quantize Q, and sage_forward_masked's mask blocks
-// (mp.prep_blocks of them) follow.  The V blocks come first so their longer row loops start early.
 // waves per SIMD the first launch asks for: 5 fit the d128 paths in 96 VGPRs (more loads in flight per CU); d256
 // holds twice the row slice and stays at the register count it needs
 template <int D> constexpr int quant_qk_waves() { return D == 256 ? 1 : 5; }
 
+// ------------------------------------------------------------------------------------------------------------------
+// V of a short key range: one workgroup owns 16 channels of one (batch, kv head) over all its keys (at most
+// V_SHORT_KEYS), so it takes their maxima and converts them from one read, held in registers (8 rows of 16 bytes per
+// thread, all loads in flight).  `base` = row 0 of the head; writes VS and V8T of the 16 channels.  Slices of 32 channels
+// hold twice the rows per thread: 1.2 us longer where few heads leave the slices on the critical path (1x8x1024x64).
+// ------------------------------------------------------------------------------------------------------------------
+constexpr int V_SHORT_KEYS = 1024;
+constexpr int V_SLICE = 16;  // channels per workgroup
+// Where one launch with V slices replaces the two with per-chunk maxima: the keys fit the registers and V is at most
+// V_SHORT_BYTES, since a slice's 32-byte row pieces use a quarter of each line they touch.  Whole call, two launches
+// against one (one MI355X, bf16): 1x8x1024x64 20.7 -> 19.6 us, 2x20x1024x64 (5 MB of V) 33.7 -> 30.8, 1x24x1024x128
+// (6 MB) 41.7 -> 39.7, 2x10x4096 queries x 77 keys x 64 22.3 -> 18.9, 1x12x8192 x 256 keys x 256 63.1 -> 58.1; past the
+// line 2x40x640x128 (13 MB) 40.8 -> 41.7, 2x40x1024x128 (21 MB) 62.4 -> 64.8.
+constexpr int64_t V_SHORT_BYTES = 8ll << 20;
+static inline bool v_short(int B, int Hkv, int Skv, int D) {
+  return Skv <= V_SHORT_KEYS && (int64_t)B * Hkv * Skv * D * 2 <= V_SHORT_BYTES;
+}
+
+template <int D, int DT>
+__device__ __forceinline__ void quant_v_slice(const uint16_t* __restrict__ base, int64_t vss, int Skv, int Skp, int slice,
+                                              float* __restrict__ vs_head, uint8_t* __restrict__ v8t_head) {
+  constexpr int ROWS = 128;                    // rows per pass: 2 threads of 8 channels each
+  constexpr int PASSES = V_SHORT_KEYS / ROWS;  // registers hold them all
+  constexpr int PITCH = V_SLICE + 4;
+  __shared__ float wave_max[4][V_SLICE];
+  __shared__ __attribute__((aligned(4))) uint8_t tile[V_SHORT_KEYS * PITCH];
+  const int c = threadIdx.x & 1, r0 = threadIdx.x >> 1;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int ch = slice * V_SLICE + 8 * c;
+  const bool has_ch = ch < D;  // D = 96: the last slices are padding, zeros
+  const uint16_t* src = base + (has_ch ? ch : 0);
+  uint4 w[PASSES];
+#pragma unroll
+  for (int g = 0; g < PASSES; g += 4) {
+    if (g * ROWS < Skv) {  // uniform
+#pragma unroll
+      for (int p = g; p < g + 4; ++p) {
+        const int row = p * ROWS + r0;
+        const bool ok = row < Skv && has_ch;
+        w[p] = load16_or_zero(src + (ok ? (int64_t)row * vss : 0), ok);
+      }
+    } else {
+#pragma unroll
+      for (int p = g; p < g + 4; ++p) w[p] = make_uint4(0, 0, 0, 0);
+    }
+  }
+  float m[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) m[i] = 0.0f;
+#pragma unroll
+  for (int p = 0; p < PASSES; ++p) {
+    const uint32_t ws[4] = {w[p].x, w[p].y, w[p].z, w[p].w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      m[2 * i] = fmaxf(m[2 * i], fabsf(elem_lo<DT>(ws[i])));
+      m[2 * i + 1] = fmaxf(m[2 * i + 1], fabsf(elem_hi<DT>(ws[i])));
+    }
+  }
+  // the rows are widened again below: the floats, kept from here, would spill
+#pragma unroll
+  for (int p = 0; p < PASSES; ++p) asm volatile("" : "+v"(w[p].x), "+v"(w[p].y), "+v"(w[p].z), "+v"(w[p].w));
+#pragma unroll
+  for (int off = 2; off < 64; off <<= 1)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) m[i] = fmaxf(m[i], __shfl_xor(m[i], off, 64));
+  if (lane < 2) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) wave_max[wave][8 * c + i] = m[i];
+  }
+  __syncthreads();
+  float cs[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float a = fmaxf(fmaxf(wave_max[0][8 * c + i], wave_max[1][8 * c + i]),
+                          fmaxf(wave_max[2][8 * c + i], wave_max[3][8 * c + i]));
+    if (r0 == 0) vs_head[ch + i] = a;
+    cs[i] = 448.0f / fmaxf(a, 1e-30f);
+  }
+#pragma unroll
+  for (int p = 0; p < PASSES; ++p) {
+    if (p * ROWS >= Skp) break;  // uniform
+    uint32_t t0, t1;
+    v_to_e4m3<DT>(w[p], cs, t0, t1);
+    uint32_t* dst = reinterpret_cast<uint32_t*>(tile + (p * ROWS + r0) * PITCH + 8 * c);
+    dst[0] = t0;
+    dst[1] = t1;
+  }
+  __syncthreads();
+  const int ksel = threadIdx.x & 63, cg = threadIdx.x >> 6;  // 64 key sets of 16, 4 groups of 4 channels
+  if (16 * ksel < Skp) v_store_set<PITCH>(tile, ksel, cg, v8t_head + (int64_t)(slice * V_SLICE + 4 * cg) * Skp, Skp);
+}
+
+// Short key ranges: one launch for all of sage_forward's quantization.  Blocks [0, nvb) own a channel slice of V each,
+// blocks [nvb, nvb + nk) quantize 64 keys of K and the rest Q.
+template <int D, int DT>
+__global__ __launch_bounds__(256, quant_qk_waves<D>()) void quant_short_kernel(
+    const uint16_t* __restrict__ x, int64_t sb, int64_t ss, int64_t sh, int H, int Sq, int row_tiles, float qs_mul,
+    int8_t* __restrict__ q8, float* __restrict__ qs, const uint16_t* __restrict__ k, int64_t ksb, int64_t kss, int64_t ksh,
+    int Skp, int nk, int8_t* __restrict__ k8, float* __restrict__ ks, const uint16_t* __restrict__ v, int64_t vsb,
+    int64_t vss, int64_t vsh, int Hkv, int Skv, float* __restrict__ vs, uint8_t* __restrict__ v8t, int nvb) {
+  const int blk = blockIdx.x;
+  if (blk < nvb) {
+    constexpr int DP = HeadDim<D>::DP, SLICES = DP / V_SLICE;
+    const int slice = blk % SLICES, bh = blk / SLICES;
+    quant_v_slice<D, DT>(v + bh / Hkv * vsb + bh % Hkv * vsh, vss, Skv, Skp, slice, vs + (int64_t)bh * DP,
+                         v8t + (int64_t)bh * DP * Skp);
+  } else if (blk < nvb + nk) {
+    quant_k_rows64<D, DT>(k, ksb, kss, ksh, Hkv, Skv, Skp, k8, ks, blk - nvb);
+  } else {
+    quant_q_rows<D, DT>(x, sb, ss, sh, H, Sq, row_tiles, qs_mul, q8, qs, blk - nvb - nk);
+  }
+}
+
+// sage_forward's first launch: blocks [0, nv) write per-chunk V maxima (vamax_chunk_rows keys each) to `vpart`,
+// blocks [nv, nv + nk) quantize 64 keys of K each, the next nq quantize Q, and sage_forward_masked's mask blocks
+// (mp.prep_blocks of them) follow.  The V blocks come first so their longer row loops start early.
 template <int D, int DT>
 __global__ __launch_bounds__(256, quant_qk_waves<D>()) void quant_qk_vamax_kernel(const uint16_t* __restrict__ x, int64_t sb, int64_t ss,
                                                              int64_t sh, int H, int Sq, int row_tiles, float qs_mul,
@@ -569,7 +694,8 @@ static void launch_quant_kv(const void* k, int64_t ksb, int64_t kss, int64_t ksh
                      Hkv, S, Skp, vs, k8, ks, v8t);
 }
 
-// sage_forward's quantization in two launches: Q, K and per-chunk V maxima, then V (reducing the maxima).
+// sage_forward's quantization: in one launch where V is small, else in two, Q, K and per-chunk V maxima, then V
+// (reducing the maxima).
 template <int D, int DT>
 static void launch_forward_quant(const void* q, int64_t qsb, int64_t qss, int64_t qsh, const void* k, int64_t ksb,
                                  int64_t kss, int64_t ksh, const void* v, int64_t vsb, int64_t vss, int64_t vsh, int B,
@@ -581,6 +707,13 @@ static void launch_forward_quant(const void* q, int64_t qsb, int64_t qss, int64_
   const int nv = vchunks * B * Hkv;
   const int nk = Skp / 64 * B * Hkv;
   const int nq = tiles * B * H;
+  if (v_short(B, Hkv, Skv, D) && mp.prep_blocks == 0) {  // a mask's ranges need the second launch
+    const int nvs = HeadDim<D>::DP / V_SLICE * B * Hkv;
+    hipLaunchKernelGGL((quant_short_kernel<D, DT>), dim3(nvs + nk + nq), dim3(256), 0, st, static_cast<const uint16_t*>(q),
+                       qsb, qss, qsh, H, Sq, tiles, qs_mul, q8, qs, static_cast<const uint16_t*>(k), ksb, kss, ksh, Skp,
+                       nk, k8, ks, static_cast<const uint16_t*>(v), vsb, vss, vsh, Hkv, Skv, vs, v8t, nvs);
+    return;
+  }
   const int nvb = Skp / 128 * B * Hkv;
   hipLaunchKernelGGL((quant_qk_vamax_kernel<D, DT>), dim3(nv + nk + nq + mp.prep_blocks), dim3(256), 0, st,
                      static_cast<const uint16_t*>(q), qsb, qss, qsh, H, Sq, tiles, qs_mul, q8, qs,
