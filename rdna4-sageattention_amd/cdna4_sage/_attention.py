@@ -19,7 +19,7 @@ _MANIFEST_PATH = Path(__file__).resolve().parent / "manifest.json"
 _MANIFEST = json.loads(_MANIFEST_PATH.read_text())
 KV_BLOCK = _MANIFEST["kv_block"]            # keys per K scale (reference: kernels/manifest.json "kv_block")
 HEAD_DIMS = tuple(_MANIFEST["head_dims"])
-LSE_HEAD_DIMS = tuple(_MANIFEST["lse"]["head_dims"])   # the LSE kernel; other head dims use the torch formula
+LSE_HEAD_DIMS = tuple(_MANIFEST["lse"]["head_dims"])   # head dims of the public lse(); return_lse takes HEAD_DIMS
 ARCHS = (_MANIFEST["arch"],)
 DTYPES = {torch.bfloat16: _capi.DTYPE_BF16, torch.float16: _capi.DTYPE_F16}
 _I32_MAX = 2**31 - 1
@@ -202,7 +202,15 @@ def _out_strides(out: torch.Tensor):
 def lse(q, k, layout="HND", sm_scale=None, is_causal=False):
     """Row logsumexp of Q K^T * scale (natural log) over the keys, fp32 [B, H, q_len], from the 16-bit inputs on the
     gfx950 LSE kernel (the value `return_lse` returns; reference: src/sageattention/core.py:23-44).  Causal masks are
-    bottom-right aligned and need q_len <= kv_len.  Raises Unsupported when the kernel cannot run these inputs."""
+    bottom-right aligned and need q_len <= kv_len.  Raises Unsupported when the kernel cannot run these inputs and for
+    head dims outside LSE_HEAD_DIMS."""
+    if q.dim() == 4 and q.shape[-1] not in LSE_HEAD_DIMS:
+        raise Unsupported("head_dim / head counts")
+    return row_lse(q, k, layout, sm_scale, is_causal)
+
+
+def row_lse(q, k, layout="HND", sm_scale=None, is_causal=False):
+    """lse for every head dim of the path (return_lse)."""
     if layout not in ("HND", "NHD"):
         raise Unsupported(f"layout {layout!r}")
     if not (q.is_cuda and k.device == q.device):
@@ -217,7 +225,7 @@ def lse(q, k, layout="HND", sm_scale=None, is_causal=False):
     else:
         B, Sq, H, D = q.shape
         Skv, Hkv = k.shape[1], k.shape[2]
-    if D not in LSE_HEAD_DIMS or k.shape[-1] != D or k.shape[0] != B or Hkv == 0 or H % Hkv:
+    if D not in HEAD_DIMS or k.shape[-1] != D or k.shape[0] != B or Hkv == 0 or H % Hkv:
         raise Unsupported("head_dim / head counts")
     if q.numel() == 0 or k.numel() == 0 or max(q.numel(), k.numel()) > _I32_MAX:
         raise Unsupported("empty or too large")

@@ -299,7 +299,8 @@ __global__ __launch_bounds__(ATT_THREADS, (attn_occupancy<layout_dim(HD), MASK =
   if (split) {  // ranges of all the keys; a causal tile may end before its last ranges, which are then empty
     const int nt = (Skv + BN - 1) / BN;
     t_lo = chunk * nt / chunks;
-    t_hi = min((chunk + 1) * nt / chunks, ntiles);
+    t_hi = (chunk + 1) * nt / chunks;
+    if (CAUSAL) t_hi = min(t_hi, ntiles);
   }
 
   // ---- mask: this lane's bit row and this wave's class row; the workgroup runs only the tiles from the first to the
@@ -686,7 +687,7 @@ __global__ __launch_bounds__(ATT_THREADS, (attn_occupancy<layout_dim(HD), MASK =
   // The first tile's K goes into the buffer the loop fills last (free until the loop's first prefetch), beside the
   // range's first tile(s).  Dense launches split only tiles of at least 8 key tiles, so without the causal flag every
   // row sees the whole first tile; a causal wave whose first row does not starts from -inf.
-  const bool seed_split = !MASK && !VARLEN && split && t_lo > 0 && t_lo < t_hi;
+  const bool seed_split = !MASK && !VARLEN && split && t_lo > 0 && (!CAUSAL || t_lo < t_hi);
   constexpr int SEED_BUF_OFS = NBUF - 1;  // buffer (t_lo + NBUF - 1) % NBUF
   if (seed_split) {
     const int8_t* kb_ = kbase;

@@ -13,6 +13,10 @@
 // max, raised only when needed: once every row of a wave has one, a tile first adds its terms with the current m and
 // keeps them when every lane's sum is below 2^16 (almost always; an overflow gives inf and fails the test), else it
 // takes the tile's max as the exact online update does.  Causal masks are bottom-right aligned (Sq <= Skv).
+//
+// Head dims 96 and 256 run it as well (96 in 128-channel LDS rows, 6 of the 8 MFMAs; 256 on 64 KiB of LDS, two
+// workgroups per CU): the fp32 torch formula they took before writes and reads every score several times
+// (1x8x4096 causal: head dim 96 1606 -> 47 us, 256 1867 -> 85 us).
 #include <type_traits>
 
 #include "sage_common.h"
@@ -48,10 +52,10 @@ template <int D, bool CAUSAL, int DT>
 __global__ __launch_bounds__(LSE_THREADS, 2) void lse_kernel(const uint16_t* __restrict__ q, int64_t qsb, int64_t qss,
                                                              int64_t qsh, const uint16_t* __restrict__ k, int64_t ksb,
                                                              int64_t kss, int64_t ksh, int H, int Hkv, int Sq,
-                                                             int Skv, int q_tiles, int total, float c,
+                                                             int Skv, int q_tiles, int total, float c, double c64,
                                                              float* __restrict__ lse) {
   constexpr int BN = LSE_BN;
-  constexpr int ROWB = D * 2;              // bytes per K row
+  constexpr int ROWB = layout_dim(D) * 2;  // bytes per K row in LDS (96 channels in rows of 128, the rest never read)
   constexpr int KCH = ROWB / 16;           // 16-byte chunks per row
   constexpr int KTILE = BN * ROWB;         // bytes per K tile
   constexpr int NK = D / 16;               // MFMAs (16 dims each) per 32-key block
@@ -98,7 +102,9 @@ __global__ __launch_bounds__(LSE_THREADS, 2) void lse_kernel(const uint16_t* __r
   for (int j = 0; j < LOADS; ++j) {
     const int L = (wave * LOADS + j) * 64 + lane;
     lrow[j] = L / KCH;
-    lchunk[j] = lse_swz<KCH>(lrow[j], L % KCH) * 8;  // in elements
+    int c = lse_swz<KCH>(lrow[j], L % KCH);
+    if (c >= D / 8) c -= D / 8;  // head dim 96: the rows' unused chunks load some chunk that exists
+    lchunk[j] = c * 8;           // in elements
     koff[j] = (uint32_t)(((int64_t)lrow[j] * kss + lchunk[j]) * 2);
   }
   // Whole tiles: the tile base pinned to an SGPR pair plus the lane's 32-bit offset (the saddr + voffset form, no
@@ -108,7 +114,7 @@ __global__ __launch_bounds__(LSE_THREADS, 2) void lse_kernel(const uint16_t* __r
     uint8_t* dst = smem[buf];
     if ((t + 1) * BN <= Skv) {
       const uint8_t* kb = reinterpret_cast<const uint8_t*>(kbase + (int64_t)t * BN * kss);
-      asm volatile("" : "+s"(kb));
+      if (D <= 128) asm volatile("" : "+s"(kb));  // (256: the compiler holds the base in VGPRs)
 #pragma unroll
       for (int j = 0; j < LOADS; ++j) {
         asm volatile("" : "+v"(koff[j]));
@@ -228,17 +234,25 @@ __global__ __launch_bounds__(LSE_THREADS, 2) void lse_kernel(const uint16_t* __r
     tile(t, std::true_type{}, t & 1);
   }
   const float lt = add_xor32_f32(l);
-  if (qvalid && hf == 0) lse[(int64_t)bh * Sq + qrow] = 0.69314718055994531f * (m * c + __log2f(lt));
+  if (qvalid && hf == 0) {
+    // ln 2 * (m * c + log2 l) rounded once: c in float64 (the terms above carry its fp32 rounding only on s - m), and
+    // log2 of l's mantissa alone in fp32.  In fp32 throughout, the three roundings made the error against float64 a
+    // quarter larger than the fp32 torch formula's (5.1e-8 to 5.9e-8 of the 2-norm against 4.1e-8 to 4.7e-8; now
+    // 3.1e-8 to 3.5e-8)
+    const int e = __builtin_amdgcn_frexp_expf(lt);
+    const float f = __log2f(__builtin_amdgcn_frexp_mantf(lt));
+    lse[(int64_t)bh * Sq + qrow] = (float)(0.69314718055994531 * ((double)m * c64 + ((double)e + (double)f)));
+  }
 }
 
 template <int D, bool CAUSAL, int DT>
 static void launch_lse(const void* q, int64_t qsb, int64_t qss, int64_t qsh, const void* k, int64_t ksb, int64_t kss,
-                       int64_t ksh, int B, int H, int Hkv, int Sq, int Skv, float c, float* lse, hipStream_t st) {
+                       int64_t ksh, int B, int H, int Hkv, int Sq, int Skv, double c, float* lse, hipStream_t st) {
   const int q_tiles = (Sq + LSE_BM - 1) / LSE_BM;
   const int total = B * H * q_tiles;
   hipLaunchKernelGGL((lse_kernel<D, CAUSAL, DT>), dim3(total), dim3(LSE_THREADS), 0, st,
                      static_cast<const uint16_t*>(q), qsb, qss, qsh, static_cast<const uint16_t*>(k), ksb, kss, ksh, H,
-                     Hkv, Sq, Skv, q_tiles, total, c, lse);
+                     Hkv, Sq, Skv, q_tiles, total, (float)c, c, lse);
 }
 
 int lse_impl(const void* q, int64_t qsb, int64_t qss, int64_t qsh, const void* k, int64_t ksb, int64_t kss,
@@ -247,7 +261,7 @@ int lse_impl(const void* q, int64_t qsb, int64_t qss, int64_t qsh, const void* k
   const char* who = "sage_lse_fwd";
   SAGE_REQUIRE(B > 0 && H > 0 && Hkv > 0 && Sq > 0 && Skv > 0, "%s: sizes must be positive", who);
   SAGE_REQUIRE(H % Hkv == 0, "%s: heads %d not a multiple of kv heads %d", who, H, Hkv);
-  if (D != 64 && D != 128) return fail(SAGE_ERR_UNSUPPORTED, "%s: head_dim %d (supported 64, 128)", who, D);
+  if (!head_dim_ok(D)) return fail(SAGE_ERR_UNSUPPORTED, "%s: head_dim %d (supported 64, 96, 128, 256)", who, D);
   if (dtype != SAGE_DTYPE_BF16 && dtype != SAGE_DTYPE_F16)
     return fail(SAGE_ERR_UNSUPPORTED, "%s: dtype code %d (bf16=0, f16=1)", who, dtype);
   if (causal && Sq > Skv) return fail(SAGE_ERR_UNSUPPORTED, "%s: causal LSE needs q_len <= kv_len", who);
@@ -259,18 +273,23 @@ int lse_impl(const void* q, int64_t qsb, int64_t qss, int64_t qsh, const void* k
   SAGE_REQUIRE((int64_t)B * H * ((Sq + LSE_BM - 1) / LSE_BM) < (1ll << 31), "%s: too many query tiles", who);
   SAGE_REQUIRE((int64_t)LSE_BN * kss < (1ll << 31), "%s: key stride too large", who);
   const double scale = sm_scale > 0.0f ? (double)sm_scale : 1.0 / __builtin_sqrt((double)D);
-  const float c = (float)(scale * 1.4426950408889634);
+  const double c = scale * 1.4426950408889634;
   hipStream_t st = (hipStream_t)stream;
 #define SAGE_LSE_CASE(DD, CC, TT) \
   launch_lse<DD, CC, TT>(q, qsb, qss, qsh, k, ksb, kss, ksh, B, H, Hkv, Sq, Skv, c, lse, st)
+#define SAGE_LSE_DIM(DD)                                                                                      \
+  do {                                                                                                        \
+    if (causal) { if (bf) SAGE_LSE_CASE(DD, true, DT_BF16); else SAGE_LSE_CASE(DD, true, DT_F16); }           \
+    else { if (bf) SAGE_LSE_CASE(DD, false, DT_BF16); else SAGE_LSE_CASE(DD, false, DT_F16); }                \
+  } while (0)
   const bool bf = dtype == SAGE_DTYPE_BF16;
-  if (D == 128) {
-    if (causal) { if (bf) SAGE_LSE_CASE(128, true, DT_BF16); else SAGE_LSE_CASE(128, true, DT_F16); }
-    else { if (bf) SAGE_LSE_CASE(128, false, DT_BF16); else SAGE_LSE_CASE(128, false, DT_F16); }
-  } else {
-    if (causal) { if (bf) SAGE_LSE_CASE(64, true, DT_BF16); else SAGE_LSE_CASE(64, true, DT_F16); }
-    else { if (bf) SAGE_LSE_CASE(64, false, DT_BF16); else SAGE_LSE_CASE(64, false, DT_F16); }
+  switch (D) {
+    case 64: SAGE_LSE_DIM(64); break;
+    case 96: SAGE_LSE_DIM(96); break;
+    case 128: SAGE_LSE_DIM(128); break;
+    default: SAGE_LSE_DIM(256); break;
   }
+#undef SAGE_LSE_DIM
 #undef SAGE_LSE_CASE
   return check_launch("lse launch");
 }

@@ -12,6 +12,7 @@ from typing import Any, Optional
 import torch
 
 import cdna4_sage
+from cdna4_sage._attention import row_lse
 
 _LSE_SCORE_BUDGET = 64 * 2**20  # fp32 scores per chunk of the LSE pass (~256 MB)
 
@@ -31,7 +32,7 @@ def _lse(q, k, tensor_layout, is_causal, sm_scale):
     the query heads that share a kv head are processed together with one fp32 batched product per row chunk."""
     _as_hnd(q, tensor_layout)  # layout check (ValueError, as the reference)
     try:
-        return cdna4_sage.lse(q, k, tensor_layout, sm_scale, is_causal)
+        return row_lse(q, k, tensor_layout, sm_scale, is_causal)
     except cdna4_sage.Unsupported:
         pass
     q, k = _as_hnd(q, tensor_layout), _as_hnd(k, tensor_layout)

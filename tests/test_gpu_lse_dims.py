@@ -1,0 +1,50 @@
+"""The logsumexp kernel at the head dims that return_lse took the fp32 torch formula for, 96 (128-channel LDS rows) and
+256, against float64: at most 2^-23 of the value (its own rounding is 2^-24) plus the scores' fp32 accumulation, on lengths
+around a tile, both layouts, strided heads, grouped heads and the causal diagonal."""
+import pytest
+import torch
+
+import cdna4_sage
+import sageattention
+from cdna4_sage._attention import row_lse
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D", [96, 256])
+@pytest.mark.parametrize("B,H,Hkv,Sq,Skv,dt,layout,causal,sm", [
+    (1, 2, 2, 1, 1, "bf16", "HND", False, None), (2, 4, 2, 33, 63, "f16", "NHD", False, 0.05),
+    (1, 4, 1, 128, 64, "bf16", "NHD", False, None), (1, 2, 2, 129, 65, "f16", "HND", False, None),
+    (1, 3, 3, 257, 1031, "bf16", "NHD", True, None), (2, 4, 2, 500, 500, "f16", "HND", True, 0.2),
+    (1, 8, 8, 1000, 1000, "bf16", "HND", True, None)])
+def test_lse_of_head_dims_96_and_256(dev, D, B, H, Hkv, Sq, Skv, dt, layout, causal, sm):
+    dtype = torch.bfloat16 if dt == "bf16" else torch.float16
+    g = torch.Generator(device=dev).manual_seed(D + Skv)
+
+    def draw(h, s):  # a slice of wider rows: neither contiguous nor without a gap between heads
+        t = torch.randn((B, s, h, D + 32) if layout == "NHD" else (B, h, s, D + 32), generator=g, device=dev)
+        return (t * 2).to(dtype)[..., 8:8 + D]
+
+    q, k = draw(H, Sq), draw(Hkv, Skv)
+    got = row_lse(q, k, layout, sm, causal)
+    qh, kh = (t if layout == "HND" else t.transpose(1, 2) for t in (q, k))
+    kt = kh.double().repeat_interleave(H // Hkv, 1).transpose(-1, -2).contiguous()
+    scale = D ** -0.5 if sm is None else sm
+    s = (qh.double() @ kt) * scale
+    # fp32 accumulation of D products, each below |q||k|: D 2^-24 of the sum of their magnitudes, and the fp32 scale
+    # of an exponent
+    bound = (qh.double().abs() @ kt.abs()).amax(-1) * scale * (D * 2.0 ** -24)
+    if causal:
+        s.masked_fill_(torch.ones(Sq, Skv, dtype=torch.bool, device=dev).triu(Skv - Sq + 1), float("-inf"))
+    ref = torch.logsumexp(s, -1)
+    assert ((got.double() - ref).abs() <= ref.abs() * 2.0 ** -23 + bound + 1e-6).all()
+    with pytest.raises(cdna4_sage.Unsupported):
+        cdna4_sage.lse(q, k, layout, sm, causal)
+
+
+def test_return_lse_uses_the_kernel(dev):
+    g = torch.Generator(device=dev).manual_seed(2)
+    q, k, v = (torch.randn(1, 16, 3000, 256, generator=g, device=dev).to(torch.bfloat16) for _ in range(3))
+    out, lse = sageattention.sageattn(q, k, v, is_causal=True, return_lse=True)
+    assert torch.equal(lse, row_lse(q, k, "HND", None, True))
+    assert torch.equal(out, sageattention.sageattn(q, k, v, is_causal=True))
