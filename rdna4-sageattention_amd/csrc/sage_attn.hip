@@ -145,8 +145,8 @@ constexpr int64_t MASK_ROW_32BIT = 1 << 26;  // 31 rows of at most this many 16-
 // PART: the format of a split tile's partials, fp16 or fp32, or (mask variants) by the argument p32.  Two kernels rather
 // than two epilogues in one: with both, the fp16 launches lost 1.4% (Flux, 158.1 -> 160.4 us; 13.8 -> 14.2 us at
 // 1x8x1024x64).
-constexpr int PART_F16 = 0, PART_F32 = 1, PART_ANY = 2;
-constexpr int part_format(bool causal, int mask) { return mask ? PART_ANY : causal ? PART_F32 : PART_F16; }
+constexpr int PART_F16 = 0, PART_F32 = 1, PART_ANY = 2, PART_NONE = 3;  // PART_NONE: no split tiles at all
+constexpr int part_format(bool causal, int mask) { return mask ? PART_ANY : causal ? PART_NONE : PART_F16; }
 template <int HD, bool CAUSAL, int OUT_DT, bool VARLEN, int MASK = MASK_NONE, int PART = part_format(CAUSAL, MASK)>
 __global__ __launch_bounds__(ATT_THREADS, (attn_occupancy<layout_dim(HD), MASK == MASK_ADD>())) void attn_kernel(
     const int8_t* __restrict__ q8, const float* __restrict__ qs, const int8_t* __restrict__ k8,
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(ATT_THREADS, (attn_occupancy<layout_dim(HD), MASK =
 
   // ---- work decode.  Dense: blocks [0, n_full) own whole query tiles (XCD-grouped; causal: longest first); each
   // later block owns one of the `chunks` key ranges of a split tile.  VARLEN: the tile table. ----
-  const bool split = !VARLEN && (int)blockIdx.x >= n_full;
+  const bool split = !VARLEN && PART != PART_NONE && (int)blockIdx.x >= n_full;
   int b, h, qt, unit = 0, chunk = 0, Sq = Sq_arg, Skv = Skv_arg;
   int64_t qrow0;       // Q8 / QS row of query 0 of this (sequence, head)
   int khead, kofs;     // K8 / KS / V8T head index and the sequence's first key row inside it
@@ -1046,14 +1046,14 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict
 //    442; d256, L 69, n 840 (768 + 72 x 3): 272 against 286; d128, L 72, n 1152 (1024 + 128 x 2): 209 against 218 with
 //    768 + 384 x 2.  Below the line: d128, L 20, n 640: 46 split, 43 whole.  More than cus / 2 tiles: d128, L 72,
 //    n 704: 146 split, 132 whole.
-//  * causal: every tile of launches of at most slots / 2 tiles, the longer the key range the more tiles (L >= n / 4
-//    at 256 CUs); past one tile per CU only where the shortest tile sees at least half the keys (chunked prefill).
-//    d128, 192 tiles of a 700-row chunk against 8192 keys (4 ranges): 80 against 120 whole; 384 tiles, 1500 rows
-//    against 9001 keys (2 ranges): 151 against 153-172; square 8 x 2048 (128 tiles, L 32): 31 against 35; below the
-//    line 16 x 2048 (256 tiles, L 32): 41 split, 36 whole; 8 x 8192 (512 tiles): 138 split, 126 whole.
+//  * causal: every tile of launches of at most cus tiles, the longer the key range the more tiles (L >= n / 4 at 256
+//    CUs).  d128, 192 tiles of a 700-row chunk against 8192 keys (4 ranges): 80 against 120 whole; square 8 x 2048
+//    (128 tiles, L 32): 31 against 35; below the line 16 x 2048 (256 tiles, L 32): 41 split, 36 whole; past one tile
+//    per CU, 384 tiles of 1500 rows against 9001 keys (2 ranges): 152 split, 149 whole, and square 8 x 8192 (512 tiles):
+//    138 split, 126 whole.
 // The tiles of the last two rules keep fp32 partials, the precision they would be accumulated in whole.
 // ------------------------------------------------------------------------------------------------------------------
-constexpr int CAUSAL_SPLIT_TILES = 512;  // no device has slots for two ranges of more causal tiles than this
+constexpr int CAUSAL_SPLIT_TILES = 256;  // causal launches of more tiles run whole on every device (its CUs at most)
 
 struct AttnPlan {
   int n_tiles, n_full, chunks;
@@ -1109,7 +1109,7 @@ static int make_plan(int B, int H, int Sq, int Skv, AttnPlan* p) {
   const int most = min(kv_tiles / 4, ATT_MAX_CHUNKS);
   int rem = 0, chunks = 1;
   if (CAUSAL) {
-    if ((int64_t)kv_tiles * cus >= 64 * (int64_t)n && (n <= cus || Skv >= 2 * (int64_t)Sq)) {
+    if (n <= cus && (int64_t)kv_tiles * cus >= 64 * (int64_t)n) {
       rem = n;
       chunks = min(slots / n, most);
       p->p32 = true;
@@ -1177,8 +1177,7 @@ static int launch_attn(const int8_t* q8, const float* qs, const int8_t* k8, cons
   uint16_t* o = static_cast<uint16_t*>(out);
   float* part = static_cast<float*>(workspace);
   auto* kernel = attn_kernel<HD, CAUSAL, OUT_DT, false>;
-  if constexpr (!CAUSAL)
-    if (p.p32) kernel = attn_kernel<HD, false, OUT_DT, false, MASK_NONE, PART_F32>;
+  if (p.p32 && n_split > 0) kernel = attn_kernel<HD, CAUSAL, OUT_DT, false, MASK_NONE, PART_F32>;
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(ATT_THREADS), 0, st, q8, qs, k8, ks, v8t, vs, o, osb, oss, osh, lse, H, Hkv,
                      Sq, Skv, kv_pad(Skv), q_tiles, p.n_tiles, p.n_full, p.chunks, (int)p.p32, part, c0, hd, VarlenTiles{},
                      MaskTabs{}, nullptr, nullptr, nullptr);
