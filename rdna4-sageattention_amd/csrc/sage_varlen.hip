@@ -201,9 +201,21 @@ __global__ __launch_bounds__(256) void varlen_prep_kernel(const int* __restrict_
         const int b = order[lo];
         const int r = (int)i - tpre[lo];
         const int nq = (cu_q[b + 1] - cu_q[b] + 127) / 128;
-        // causal: the sequence's tiles longest first across its heads (its last query tile of every head, then the one
-        // before, ...), so that its short tiles come last; otherwise head by head
-        e = causal ? make_int4(b, r % H, nq - 1 - r / H, 0) : make_int4(b, r / nq, r % nq, 0);
+        // Within a sequence each XCD takes its own share of the heads, whose K8 / V8T stay in its L2, as in the dense
+        // launches (a sequence's blocks may start on any XCD: that only renames them); causal: longest first across
+        // an XCD's heads, or, where the heads do not divide over the XCDs, across all of them.
+        int h, qt;
+        if (!causal) {
+          const int logical = xcd_remap(r, H * nq);
+          h = logical / nq;
+          qt = logical % nq;
+        } else if (H % 8 == 0) {
+          causal_tile(r, H, nq, h, qt);
+        } else {
+          h = r % H;
+          qt = nq - 1 - r / H;
+        }
+        e = make_int4(b, h, qt, 0);
       }
       tiles[i] = e;
     }
