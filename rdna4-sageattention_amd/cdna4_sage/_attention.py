@@ -239,7 +239,7 @@ def row_lse(q, k, layout="HND", sm_scale=None, is_causal=False):
     k, sk_ = _bsh(k, layout)
     out = torch.empty((B, H, Sq), device=q.device, dtype=torch.float32)
     with torch.cuda.device(q.device):
-        _capi.call("sage_lse_fwd", _ptr(q), *sq_, _ptr(k), *sk_, B, H, Hkv, Sq, Skv, D, DTYPES[q.dtype],
+        _capi.call("sage_row_lse_fwd", _ptr(q), *sq_, _ptr(k), *sk_, B, H, Hkv, Sq, Skv, D, DTYPES[q.dtype],
                    int(bool(is_causal)), float(sm_scale or 0.0), _ptr(out), torch.cuda.current_stream(q.device).cuda_stream)
     return out
 

@@ -257,8 +257,7 @@ static void launch_lse(const void* q, int64_t qsb, int64_t qss, int64_t qsh, con
 
 int lse_impl(const void* q, int64_t qsb, int64_t qss, int64_t qsh, const void* k, int64_t ksb, int64_t kss,
              int64_t ksh, int B, int H, int Hkv, int Sq, int Skv, int D, int dtype, int causal, float sm_scale,
-             float* lse, void* stream) {
-  const char* who = "sage_lse_fwd";
+             float* lse, void* stream, const char* who) {
   SAGE_REQUIRE(B > 0 && H > 0 && Hkv > 0 && Sq > 0 && Skv > 0, "%s: sizes must be positive", who);
   SAGE_REQUIRE(H % Hkv == 0, "%s: heads %d not a multiple of kv heads %d", who, H, Hkv);
   if (!head_dim_ok(D)) return fail(SAGE_ERR_UNSUPPORTED, "%s: head_dim %d (supported 64, 96, 128, 256)", who, D);
@@ -296,9 +295,24 @@ int lse_impl(const void* q, int64_t qsb, int64_t qss, int64_t qsh, const void* k
 
 }  // namespace sage
 
-extern "C" int sage_lse_fwd(const void* q, int64_t qsb, int64_t qss, int64_t qsh, const void* k, int64_t ksb,
-                            int64_t kss, int64_t ksh, int B, int H, int Hkv, int Sq, int Skv, int D, int dtype,
-                            int causal, float sm_scale, float* lse, void* stream) {
+extern "C" {
+
+int sage_lse_fwd(const void* q, int64_t qsb, int64_t qss, int64_t qsh, const void* k, int64_t ksb, int64_t kss,
+                 int64_t ksh, int B, int H, int Hkv, int Sq, int Skv, int D, int dtype, int causal, float sm_scale,
+                 float* lse, void* stream) {
   sage::clear_error();
-  return sage::lse_impl(q, qsb, qss, qsh, k, ksb, kss, ksh, B, H, Hkv, Sq, Skv, D, dtype, causal, sm_scale, lse, stream);
+  if (D != 64 && D != 128)
+    return sage::fail(SAGE_ERR_UNSUPPORTED, "sage_lse_fwd: head_dim %d (supported 64, 128)", D);
+  return sage::lse_impl(q, qsb, qss, qsh, k, ksb, kss, ksh, B, H, Hkv, Sq, Skv, D, dtype, causal, sm_scale, lse, stream,
+                        "sage_lse_fwd");
 }
+
+int sage_row_lse_fwd(const void* q, int64_t qsb, int64_t qss, int64_t qsh, const void* k, int64_t ksb, int64_t kss,
+                     int64_t ksh, int B, int H, int Hkv, int Sq, int Skv, int D, int dtype, int causal, float sm_scale,
+                     float* lse, void* stream) {
+  sage::clear_error();
+  return sage::lse_impl(q, qsb, qss, qsh, k, ksb, kss, ksh, B, H, Hkv, Sq, Skv, D, dtype, causal, sm_scale, lse, stream,
+                        "sage_row_lse_fwd");
+}
+
+}  // extern "C"

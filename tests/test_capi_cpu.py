@@ -270,3 +270,18 @@ def test_bench_intermediates_have_the_abi_layout_sizes():
                 4 * B * Hkv * dl]
         got = [t.numel() * t.element_size() for t in bench.intermediates(cfg, "meta")]
         assert got == want, (name, got, want)
+
+
+def test_lse_entries_head_dims():
+    """sage_lse_fwd takes head dims 64 and 128; sage_row_lse_fwd, which return_lse uses, those of the attention."""
+    lib = _capi.lib()
+    shape = (1, 4, 2, 64, 64)
+
+    def call(entry, D):
+        return getattr(lib, entry)(P, 0, 128, 0, P, 0, 128, 0, *shape, D, 9, 0, 0.0, P, None)
+
+    for D in (96, 256, 80):
+        assert call("sage_lse_fwd", D) == _capi.SAGE_ERR_UNSUPPORTED and "head_dim" in _err()
+    assert call("sage_row_lse_fwd", 80) == _capi.SAGE_ERR_UNSUPPORTED and "head_dim" in _err()
+    for D in (96, 256):  # past the head dims: the dtype code
+        assert call("sage_row_lse_fwd", D) == _capi.SAGE_ERR_UNSUPPORTED and "dtype" in _err()

@@ -6,6 +6,7 @@ import torch
 
 import cdna4_sage
 import sageattention
+from sageattention import core
 from cdna4_sage._attention import row_lse
 
 pytestmark = pytest.mark.gpu
@@ -48,3 +49,21 @@ def test_return_lse_uses_the_kernel(dev):
     out, lse = sageattention.sageattn(q, k, v, is_causal=True, return_lse=True)
     assert torch.equal(lse, row_lse(q, k, "HND", None, True))
     assert torch.equal(out, sageattention.sageattn(q, k, v, is_causal=True))
+
+
+@pytest.mark.parametrize("D", [96, 256])
+def test_return_lse_with_gradients_keeps_the_torch_formula(dev, D):
+    g = torch.Generator(device=dev).manual_seed(D)
+    q, k = (torch.randn(1, 2, 70, D, generator=g, device=dev).to(torch.bfloat16).requires_grad_() for _ in range(2))
+    lse = core._lse(q, k, "HND", True, None)
+    lse.sum().backward()
+    with torch.no_grad():
+        # both are within 1e-6 of float64 in the 2-norm
+        assert (core._lse(q, k, "HND", True, None) - lse).norm() <= 2e-6 * lse.norm()
+    qd, kd = (t.detach().double().requires_grad_() for t in (q, k))
+    s = (qd @ kd.transpose(-1, -2).contiguous()) * D ** -0.5
+    s = s.masked_fill(torch.ones(70, 70, dtype=torch.bool, device=dev).triu(1), float("-inf"))
+    torch.logsumexp(s, -1).sum().backward()
+    for got, want in ((q.grad, qd.grad), (k.grad, kd.grad)):
+        # the gradient's own bf16 rounding, 2^-9 an element
+        assert (got.double() - want).norm() <= 2.0 ** -8 * want.norm()
