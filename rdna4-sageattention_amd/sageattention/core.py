@@ -15,6 +15,7 @@ import cdna4_sage
 from cdna4_sage._attention import row_lse
 
 _LSE_SCORE_BUDGET = 64 * 2**20  # fp32 scores per chunk of the LSE pass (~256 MB)
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
 def _as_hnd(t: torch.Tensor, tensor_layout: str) -> torch.Tensor:
@@ -31,8 +32,11 @@ def _lse(q, k, tensor_layout, is_causal, sm_scale):
     computes it (16-bit products exact in fp32, fp32 accumulation); elsewhere, and for shapes the kernel does not take,
     the query heads that share a kv head are processed together with one fp32 batched product per row chunk."""
     _as_hnd(q, tensor_layout)  # layout check (ValueError, as the reference)
+    # head dims outside LSE_HEAD_DIMS keep the torch formula where it is traced or differentiated
+    plain = (type(q) in _PLAIN and type(k) in _PLAIN and not torch.compiler.is_compiling()
+             and not (torch.is_grad_enabled() and (q.requires_grad or k.requires_grad)))
     try:
-        return row_lse(q, k, tensor_layout, sm_scale, is_causal)
+        return (row_lse if plain else cdna4_sage.lse)(q, k, tensor_layout, sm_scale, is_causal)
     except cdna4_sage.Unsupported:
         pass
     q, k = _as_hnd(q, tensor_layout), _as_hnd(k, tensor_layout)
