@@ -137,7 +137,7 @@ def sageattn_varlen(
     read back, or with CDNA4_SAGE_VARLEN_ROUTE=0, the packed pass takes every sequence (no host synchronisation; the
     short ones are then quantized too).  Without a gfx950 GPU, or when the longest key sequence is below MIN_KV, every
     sequence goes through sageattn; empty query sequences are skipped."""
-    mq, mk = _int_or_none(max_seqlen_q), _int_or_none(max_seqlen_k)
+    mk = _int_or_none(max_seqlen_k)
     if q.is_cuda and (mk is None or mk >= cdna4_sage.MIN_KV):
         sync_free = (not cdna4_sage.VARLEN_ROUTE or torch.compiler.is_compiling()
                      or torch.cuda.is_current_stream_capturing())
@@ -145,8 +145,11 @@ def sageattn_varlen(
             if sync_free:
                 return cdna4_sage.attention_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
                                                    sm_scale=sm_scale, is_causal=is_causal)
-            if cu_seqlens_q.device == q.device and cu_seqlens_k.device == q.device:
-                out = _varlen_overlapped(q, k, v, cu_seqlens_q, cu_seqlens_k, mq, mk, is_causal, sm_scale)
+            # by the caller's maximum lengths (plain numbers) some sequence may take the kernel: no wait for the offsets
+            if (cu_seqlens_q.device == q.device and cu_seqlens_k.device == q.device
+                    and isinstance(max_seqlen_q, int) and mk is not None
+                    and _kernel_takes(max_seqlen_q, mk, q.shape[1], is_causal)):
+                out = _varlen_overlapped(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, mk, is_causal, sm_scale)
                 if out is not None:
                     return out
             else:
@@ -177,12 +180,9 @@ def _int_or_none(x):
 def _varlen_overlapped(q, k, v, cu_seqlens_q, cu_seqlens_k, max_q, max_k, is_causal, sm_scale):
     """The routed packed call with the offsets on the GPU: the packed pass is queued before they are read back, and
     the side stream reads them and runs the sequences that take torch SDPA beside it, so the GPU neither waits for the
-    host nor runs those short, few-workgroup calls alone.  None when no sequence takes the kernel: by the caller's
-    maximum lengths before anything is queued, else after the offsets are read (the pass's output is then dropped).
-    Six sequences of 640 (SDPA) to 4608 tokens, 24 heads x 128: 658 -> 575 us per call."""
-    if max_q is not None and max_k is not None and \
-            q.shape[1] * max_q * max_k // (2 if is_causal else 1) < cdna4_sage.MIN_WORK:
-        return None
+    host nor runs those short, few-workgroup calls alone.  None when the offsets hold no sequence that takes the kernel
+    (the pass's output is then dropped).  Six sequences of 640 (SDPA) to 4608 tokens, 24 heads x 128: 658 -> 575 us per
+    call."""
     cur, side = torch.cuda.current_stream(q.device), _side_stream(q.device)
     side.wait_stream(cur)  # the inputs, the offsets among them
     out = cdna4_sage.attention_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_q, max_k, sm_scale=sm_scale,
@@ -195,9 +195,9 @@ def _varlen_overlapped(q, k, v, cu_seqlens_q, cu_seqlens_k, max_q, max_k, is_cau
         rest = [s for s, f in zip(seqs, fast) if not f]
         if not rest:
             return out
+        for t in (q, k, v):
+            t.record_stream(side)
         parts = [_one_sequence(q, k, v, *s, is_causal, sm_scale) for s in rest]
-    for t in (q, k, v):
-        t.record_stream(side)
     cur.wait_stream(side)
     for (q0, q1, _, _), part in zip(rest, parts):
         out[q0:q1] = part

@@ -5,6 +5,7 @@ lengths promise a kernel sequence that the offsets do not hold."""
 import pytest
 import torch
 
+import cdna4_sage
 import sageattention
 
 pytestmark = pytest.mark.gpu
@@ -48,3 +49,25 @@ def test_offsets_on_the_gpu_give_the_same_bits(dev, lens, H, D, causal, claim):
                 same = torch.equal(got, want)
                 del churn
             assert same, (seed, s)
+
+
+def test_lengths_that_are_not_plain_numbers(dev):
+    """Maximum query lengths on the GPU, or none: never read back, so the call can be captured, and the results are those
+    of plain numbers."""
+    q, k, v, ends = _batch(dev, [3000, 500, 2900], 8, 128, torch.bfloat16, 7)
+    cu = ends.to(dev)
+    on_gpu = torch.tensor(3000, device=dev)
+    want = sageattention.sageattn_varlen(q, k, v, ends, ends, 3000, 3000)
+    for mq in (on_gpu, None, 1):
+        assert torch.equal(sageattention.sageattn_varlen(q, k, v, cu, cu, mq, 3000), want)
+    packed = cdna4_sage.attention_varlen(q, k, v, cu, cu)
+    torch.cuda.synchronize(dev)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = sageattention.sageattn_varlen(q, k, v, cu, cu, on_gpu, 3000)
+    for _ in range(3):
+        noise = torch.randn(1 << 20, device=dev)
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize(dev)
+        assert torch.equal(out, packed) and torch.isfinite(noise).all()
