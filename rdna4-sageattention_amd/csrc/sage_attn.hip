@@ -1039,19 +1039,26 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict
 //    tiles, over slots / (n mod slots) ranges; fp16 partials, the most ranges for the least traffic.  d128, L 72,
 //    n 864 (768 + 96 x 8): 165 against 204 whole; with L < 48 the merge costs more than it gains (d128, L 20, n 288:
 //    42 split, 31 whole; d64, L 14, n 448: 29.5 split, 19.7 whole; d64, L 64, n 1536 over 2 ranges: 176 split, 161
-//    whole).
+//    whole).  Three ranges as well where the round has at most 3/4 of a tile per CU (whole calls at d256, n 660,
+//    512 + 148 x 3: L 64 264 against 279 whole, L 512 1754 against 1997) or L >= 112 (n 1024, 768 + 256 x 3: d128
+//    L 64 213 against 205 whole, L 128 385 against 383, L 512 1433 against 1465; d96 L 512 1204 against 1252; d128,
+//    n 10240, L 512 11721 against 11894; d64, n 1344, 1024 + 320 x 3: L 128 298 against 305 with 1280 + 64 x 4).
 //  * else the tiles past the last full multiple of cus, at most cus / 2 of them and L >= 32 (20 past the first
 //    round), over cus / that many ranges: one more unit for every CU instead of one more tile for some.  d64, L 64,
 //    n 640 (512 + 128 x 2): 73 against 86 whole; d128, L 72, n 576: 113 against 122; d128, L 265, n 640: 403 against
 //    442; d256, L 69, n 840 (768 + 72 x 3): 272 against 286; d128, L 72, n 1152 (1024 + 128 x 2): 209 against 218 with
 //    768 + 384 x 2.  Below the line: d128, L 20, n 640: 46 split, 43 whole.  More than cus / 2 tiles: d128, L 72,
 //    n 704: 146 split, 132 whole.
+//  * else two ranges of the last round where L >= 128 and the round leaves CUs without a tile, or without the second
+//    (whole calls): d256, n 768 (512 + 256 x 2), L 96 391 against 388 whole, L 192 716 against 736, L 512 1809 against
+//    1905; d64, n 448, L 64 81 against 78, L 128 136 against 138, L 512 460 against 497; d64, n 1440 (1024 + 416 x 2),
+//    L 256 662 against 672.  Not two full tiles per CU: d64, n 1536, L 512 1307 split, 1275 whole.  fp16 partials.
 //  * causal: every tile of launches of at most cus tiles, the longer the key range the more tiles (L >= n / 4 at 256
 //    CUs).  d128, 192 tiles of a 700-row chunk against 8192 keys (4 ranges): 80 against 120 whole; square 8 x 2048
 //    (128 tiles, L 32): 31 against 35; below the line 16 x 2048 (256 tiles, L 32): 41 split, 36 whole; past one tile
 //    per CU, 384 tiles of 1500 rows against 9001 keys (2 ranges): 152 split, 149 whole, and square 8 x 8192 (512 tiles):
 //    138 split, 126 whole.
-// The tiles of the last two rules keep fp32 partials, the precision they would be accumulated in whole.
+// The tiles of the second and the causal rule keep fp32 partials, the precision they would be accumulated in whole.
 // ------------------------------------------------------------------------------------------------------------------
 constexpr int CAUSAL_SPLIT_TILES = 256;  // causal launches of more tiles run whole on every device (its CUs at most)
 
@@ -1117,15 +1124,21 @@ static int make_plan(int B, int H, int Sq, int Skv, AttnPlan* p) {
   } else {
     const int rem_round = n % slots, rem_cu = n % cus;
     const bool past_one = n >= 2 * cus;  // every CU has at least two tiles
-    if (n <= cus || (rem_round > 0 && slots / rem_round >= (past_one ? 4 : 2) && kv_tiles >= 48 &&
-                     (past_one || 2 * rem_cu <= cus))) {
+    const int ranges = rem_round > 0 ? slots / rem_round : 1;
+    const bool round = past_one ? ranges >= 4 || (ranges == 3 && (4 * rem_round <= 3 * cus || kv_tiles >= 112))
+                                : ranges >= 2 && 2 * rem_cu <= cus;
+    if (n <= cus || (round && kv_tiles >= 48)) {
       rem = rem_round;
-      chunks = rem > 0 ? min(slots / rem, most) : 1;
+      chunks = rem > 0 ? min(ranges, most) : 1;
     } else if (rem_cu > 0 && (past_one ? 2 * rem_cu <= cus && kv_tiles >= (n > slots ? 20 : 32)
                                        : 4 * rem_cu <= cus && kv_tiles >= 48)) {
       rem = rem_cu;
       chunks = min(cus / rem, most);
       p->p32 = true;
+    } else if (ranges >= 2 && kv_tiles >= 128 && (rem_round <= cus || 4 * rem_cu <= 3 * cus) &&
+               (rem_round <= cus || rem_cu > 0)) {
+      rem = rem_round;
+      chunks = min(ranges, most);
     }
   }
   if (chunks < 2) return SAGE_OK;

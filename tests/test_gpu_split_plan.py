@@ -113,3 +113,37 @@ def test_noalloc_runs_whole_where_only_the_partials_do_not_fit(dev):
                code, None, None, 0, torch.cuda.current_stream(dev).cuda_stream)
     torch.cuda.synchronize(dev)
     assert torch.equal(out, whole)
+
+
+@pytest.mark.parametrize("B,H,Sq,L,D,n_full,chunks", [
+    (1, 22, 3840, 47, 256, 660, 1), (1, 22, 3840, 48, 256, 512, 3),        # 148 tiles in the last round: three ranges
+    (1, 32, 4096, 111, 128, 1024, 1), (1, 32, 4096, 112, 128, 768, 3),     # a tile for every CU in it
+    (1, 21, 8192, 111, 64, 1280, 4), (1, 21, 8192, 112, 64, 1024, 3),      # fp32 past the CUs before, 320 tiles after
+    (1, 12, 8192, 127, 256, 768, 1), (1, 12, 8192, 128, 256, 512, 2),      # two ranges
+    (1, 14, 4096, 127, 64, 448, 1), (1, 14, 4096, 128, 64, 0, 2),
+    (1, 24, 8192, 512, 64, 1536, 1),                                        # two full tiles per CU: whole
+    (1, 40, 32760, 512, 128, 9984, 3),
+])
+def test_plan_of_long_walks(dev, B, H, Sq, L, D, n_full, chunks):
+    full, ch, ws = _capi.attn_plan(dev.index or 0, B, H, Sq, L * 64, D, 0)
+    assert (full, ch) == (n_full, chunks)
+    rem = B * H * ((Sq + 127) // 128) - full
+    assert ws == (rem * ch * 128 * ((4 if ch == 4 else 2) * D + 8) if ch > 1 else 0)
+
+
+def test_three_ranges_of_head_dim_256_against_whole_tiles(dev):
+    B, H, Sq, Skv, D, dt = 1, 22, 3801, 3067, 256, BF16
+    full, ch, ws = _capi.attn_plan(dev.index or 0, B, H, Sq, Skv, D, 0)
+    assert (full, ch) == (512, 3)
+    t, code = _quantized(dev, B, H, H, Sq, Skv, D, dt, seed=11)
+    outs = []
+    for size in (0, ws):
+        out = torch.full((B, Sq, H, D), float("nan"), device=dev, dtype=dt)
+        buf = torch.full((max(size, 4) // 4,), float("nan"), device=dev)
+        _capi.call("sage_attn_fwd", *(x.data_ptr() for x in t), out.data_ptr(), *out.stride()[:3], B, H, H, Sq, Skv, D, 0,
+                   code, None, buf.data_ptr() if size else None, size, torch.cuda.current_stream(dev).cuda_stream)
+        torch.cuda.synchronize(dev)
+        outs.append(out.double())
+    whole, split = outs
+    # the same probabilities: the fp16 partials' rounding (2^-11) and the output's own (2^-9, twice)
+    assert (split - whole).norm() <= 2.0 ** -8 * whole.norm()
