@@ -626,10 +626,15 @@ def fp32_partials(rows, chunks: int, seq_kv: int, head_dim: int, causal: bool) -
         return False
     n, n_full = rows.plan
     cus, slots = 256, 256 * {64: 4, 96: 3, 128: 3, 256: 2}[head_dim]
-    rem = n % slots
-    rounds = n <= cus or (rem > 0 and slots // rem >= (4 if n >= 2 * cus else 2) and (seq_kv + 63) // 64 >= 48
-                          and (n >= 2 * cus or 2 * (n % cus) <= cus))
-    return not rounds
+    kv_tiles, rem, rem_cu = (seq_kv + 63) // 64, n % slots, n % cus
+    ranges = slots // rem if rem else 1
+    if n >= 2 * cus:
+        short_round = ranges >= 4 or (ranges == 3 and (4 * rem <= 3 * cus or kv_tiles >= 112))
+    else:
+        short_round = ranges >= 2 and 2 * rem_cu <= cus
+    if n <= cus or (short_round and kv_tiles >= 48):
+        return False
+    return n - n_full == rem_cu and 2 * rem_cu <= cus   # else two ranges of the last round
 
 
 def round_output(x: np.ndarray, out_dtype: str) -> np.ndarray:
