@@ -10,6 +10,7 @@ kernels.
 from typing import Any, Optional
 
 import torch
+from torch.autograd import forward_ad
 
 import cdna4_sage
 from cdna4_sage._attention import row_lse
@@ -26,17 +27,26 @@ def _as_hnd(t: torch.Tensor, tensor_layout: str) -> torch.Tensor:
     raise ValueError(f"tensor_layout must be 'HND' or 'NHD', got {tensor_layout!r}")
 
 
+def _plain_call(*ts) -> bool:
+    """Whether a call on these tensors is carried out now and seen by nobody else: no torch.compile, export, jit.trace or
+    dispatch mode (make_fx and the like) records it, no subclass or functorch transform (vmap, jvp, grad) holds the
+    tensors, and neither reverse- nor forward-mode autograd follows them."""
+    if (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0
+            or (torch.is_grad_enabled() and any(t.requires_grad for t in ts))):
+        return False
+    return all(type(t) in _PLAIN and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+               and forward_ad.unpack_dual(t).tangent is None for t in ts)
+
+
 def _lse(q, k, tensor_layout, is_causal, sm_scale):
     """Row logsumexp of Q K^T * scale over the keys, fp32 [B, H, q_len], on the unquantized inputs
     (reference: src/sageattention/core.py:23-44).  Causal masks are bottom-right aligned.  On gfx950 the LSE kernel
     computes it (16-bit products exact in fp32, fp32 accumulation); elsewhere, and for shapes the kernel does not take,
     the query heads that share a kv head are processed together with one fp32 batched product per row chunk."""
     _as_hnd(q, tensor_layout)  # layout check (ValueError, as the reference)
-    # head dims outside LSE_HEAD_DIMS keep the torch formula where it is traced or differentiated
-    plain = (type(q) in _PLAIN and type(k) in _PLAIN and not torch.compiler.is_compiling()
-             and not (torch.is_grad_enabled() and (q.requires_grad or k.requires_grad)))
+    # head dims outside LSE_HEAD_DIMS keep the torch formula where a tracer, a transform or autograd has to see it
     try:
-        return (row_lse if plain else cdna4_sage.lse)(q, k, tensor_layout, sm_scale, is_causal)
+        return (row_lse if _plain_call(q, k) else cdna4_sage.lse)(q, k, tensor_layout, sm_scale, is_causal)
     except cdna4_sage.Unsupported:
         pass
     q, k = _as_hnd(q, tensor_layout), _as_hnd(k, tensor_layout)
