@@ -134,8 +134,8 @@ __global__ __launch_bounds__(LSE_THREADS, 2) void lse_kernel(const uint16_t* __r
   for (int i = 0; i < NK; ++i) ko[i] = ln * ROWB + lse_swz<KCH>(ln, 2 * i + hf) * 16;
 
   float m = -INFINITY, l = 0.0f;
-  float negm = 0.0f;    // -(m * c) once m is finite
-  bool fastok = false;  // every row of the wave has a finite m: tiles start with the current m
+  float negm = 0.0f;    // -(m * c) of such an m
+  bool fastok = false;  // every row of the wave has an m below 2^24: tiles start with the current m
   // One tile: S^T from the LDS buffer, the MASKED body clears keys past Skv and (causal) past the row's diagonal.
   // The two bodies sit in two loops (tiles before t_mask need no mask for any row of the wave): with the mask test
   // in one loop the compiler turns the masking into compares and selects on every tile.
@@ -186,21 +186,28 @@ __global__ __launch_bounds__(LSE_THREADS, 2) void lse_kernel(const uint16_t* __r
 #pragma unroll
       for (int v = 0; v < 16; ++v) mx = fmaxf(mx, sv[1][v]);
       mx = max_xor32_f32(mx);
-      const float m_new = fmaxf(m, mx);
-      const float corr = __builtin_amdgcn_exp2f((m - m_new) * c);  // m = -inf on the first tile: corr = 0
-      const float neg = 0.0f - m_new * c;
+      // The terms are 2^(s * c - m * c) with m * c rounded once.  Where that rounding is more than a unit (m * c past 2^24)
+      // m is subtracted from the scores first.  An infinite max (infinite scores, or scores that overflow with c) is no
+      // reference at all: its terms are taken against 0, so that such a row ends as inf, -inf or (a NaN among its scores)
+      // NaN, as torch.logsumexp gives.
+      float m_new = fmaxf(m, mx);
+      const float mc = m_new * c;
+      const bool finite = fabsf(mc) < INFINITY, small = fabsf(mc) < 0x1p24f;
+      m_new = finite ? m_new : mc;
+      const float corr = m == m_new ? 1.0f : __builtin_amdgcn_exp2f((m - m_new) * c);  // m = -inf (first tile): corr = 0
+      const float ref = finite && !small ? m_new : 0.0f, neg = small ? 0.0f - mc : 0.0f;
       float ps[4];
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[kb][v], c, neg));
+          const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[kb][v] - ref, c, neg));
           ps[v & 3] = (kb == 0 && v < 4) ? e : ps[v & 3] + e;
         }
       l = l * corr + ((ps[0] + ps[1]) + (ps[2] + ps[3]));
       m = m_new;
-      negm = m == -INFINITY ? 0.0f : neg;  // a row with no visible key yet keeps m = -inf
-      fastok = __ballot(m == -INFINITY) == 0;
+      negm = neg;
+      fastok = __ballot(!small) == 0;  // (a row with no visible key yet keeps m = -inf)
     }
     // the wait for the next tile's direct loads comes after this tile's arithmetic (l is its last result; without
     // the operand the scheduler may hoist the wait into the middle of the tile)

@@ -67,3 +67,40 @@ def test_return_lse_with_gradients_keeps_the_torch_formula(dev, D):
     for got, want in ((q.grad, qd.grad), (k.grad, kd.grad)):
         # the gradient's own bf16 rounding, 2^-9 an element
         assert (got.double() - want).norm() <= 2.0 ** -8 * want.norm()
+
+
+@pytest.mark.parametrize("D", [64, 96, 128, 256])
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("causal", [False, True])
+def test_lse_of_infinite_scores_is_the_formula_s(dev, D, dt, causal):
+    """Rows with infinite or very large scores (from infinite inputs, from products past fp32, of one sign or both, in the first key tile or
+    a later one) and with NaN: infinite or NaN exactly where torch.logsumexp of the scores is, the other rows as always."""
+    dtype = torch.bfloat16 if dt == "bf16" else torch.float16
+    g = torch.Generator(device=dev).manual_seed(D)
+    S, inf = 200, float("inf")
+    q, k = (torch.randn(1, 3, S, D, generator=g, device=dev) for _ in range(2))
+    q[..., 0] = 0.0                     # channel 0 meets the keys below in the rows that set it
+    k[..., 0] = 1.0
+    q[0, :, 3, 0] = q[0, :, 150, 0] = inf
+    q[0, :, 40, 0] = q[0, :, 199, 0] = -inf
+    k[0, 1, 70, 0] = -1.0               # head 1: one score of the other sign
+    k[0, 2, 71, 0] = 0.0                # head 2: one NaN
+    q[0, 0, 100, 5] = float("nan")
+    # scores so large that the rounding of one in fp32 is far above the terms' exponents (f16: 65000 x 65000)
+    q[0, :, 20:24, 0] = torch.tensor([1.0, -1.0, 1.0, -1.0], device=dev) * (1e9 if dt == "bf16" else 65000.0)
+    k[0, 0, 10:13, 0] = 3e9 if dt == "bf16" else 65000.0
+    if dt == "bf16":                    # products past the largest fp32
+        q[0, 0, 60:64, 0] = torch.tensor([1e30, -1e30, 1e30, -1e30], device=dev)
+        k[0, 0, 90:94, 0] = 1e30
+    q, k = q.to(dtype), k.to(dtype)
+    got = row_lse(q, k, "HND", None, causal)
+    s = (q.float() @ k.float().transpose(-1, -2).contiguous()) * D ** -0.5
+    if causal:
+        s.masked_fill_(torch.ones(S, S, dtype=torch.bool, device=dev).triu(1), -inf)
+    want = torch.logsumexp(s, -1)
+    assert int((want == inf).sum()) >= 2 and int((want == -inf).sum()) >= 2 and int(want.isnan().sum()) >= 2
+    assert torch.equal(got.isnan(), want.isnan())
+    odd = want.isinf()
+    assert torch.equal(got[odd], want[odd])
+    rest = want.isfinite()
+    torch.testing.assert_close(got[rest], want[rest], atol=1e-5, rtol=1e-6)
