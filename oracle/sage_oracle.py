@@ -295,7 +295,7 @@ def attention(q8, qs, k8, ks, v8, vs, seq_kv: int, causal: bool = False, block_n
     (m_c, l_c, fp16(O_c / l_c)) and merged with M = max m_c, W_c = exp2((m_c - M) * cl) * l_c, L = sum W_c,
     O = sum W_c * fp16(O_c / l_c) (float32, chunk order), then the usual epilogue with L.  A range in which a row
     sees no key (l_c = 0, m_c = -inf) stores 0 and weighs 0.  Plans whose partials the kernel stores in fp32
-    (``fp32_partials``) skip the fp16 rounding.  Causal calls without a mask: a row's later ranges start from the
+    (``split_rows(fp32=True)``) skip the fp16 rounding.  Causal calls without a mask: a row's later ranges start from the
     max after tile 0 only where the first row of its 32-row group sees all of that tile.
 
     ``attn_mask``: bool array broadcastable to [B, H, Sq, seq_kv], True where the query attends the key (the
@@ -350,7 +350,7 @@ def attention(q8, qs, k8, ks, v8, vs, seq_kv: int, causal: bool = False, block_n
         chunks, rows = kv_split
         # the kernel's seed: a range that starts after the first kernel tile its 128-row block visits starts from the
         # walk's running max after that tile, instead of from -inf (no mask: tile 0)
-        fp32 = fp32_partials(rows, chunks, seq_kv, D, causal and attn_mask is None)
+        fp32 = getattr(rows, "fp32", False)
         first, m_seed = _seed_tiles(q8, cl, k8, ks, v8, seq_kv, causal, block_n, threshold, attn_mask, qpos, wide)
         parts = []
         for c in range(chunks):
@@ -595,46 +595,34 @@ def _bias_groups(attn_mask, seq_kv, causal, causal_off, kt):
     return grp[:, :, np.arange(Sq) // 32]
 
 
-def split_rows(B: int, H_total: int, Sq: int, n_full: int, heads=None, block_m: int = 128) -> np.ndarray:
+def split_rows(B: int, H_total: int, Sq: int, n_full: int, heads=None, block_m: int = 128,
+               fp32: bool = False) -> np.ndarray:
     """Bool [B, len(heads), Sq]: rows of the query tiles numbered >= n_full, where the gfx950 kernel numbers the
     tile of row r of batch b, head h as (b * H_total + h) * ceil(Sq / block_m) + r // block_m.  ``heads`` lists the
-    heads of a sample by their index in the full problem (default: all H_total heads)."""
+    heads of a sample by their index in the full problem (default: all H_total heads); ``fp32``: the format of the plan's
+    partials (``plan_fp32``)."""
     heads = np.arange(H_total) if heads is None else np.asarray(heads)
     q_tiles = (Sq + block_m - 1) // block_m
     tile = ((np.arange(B)[:, None, None] * H_total + heads[None, :, None]) * q_tiles
             + (np.arange(Sq) // block_m)[None, None, :])
     rows = (tile >= n_full).view(_SplitRows)
-    rows.plan = (B * H_total * q_tiles, n_full)
+    rows.fp32 = bool(fp32)
     return rows
 
 
 class _SplitRows(np.ndarray):
-    """split_rows' array with the plan it came from, (query tiles, whole tiles), which its slices keep."""
-    plan = None
+    """split_rows' array with the format of the plan's partials, which its slices keep."""
+    fp32 = False
 
     def __array_finalize__(self, obj):
-        self.plan = getattr(obj, "plan", None)
+        self.fp32 = getattr(obj, "fp32", False)
 
 
-def fp32_partials(rows, chunks: int, seq_kv: int, head_dim: int, causal: bool) -> bool:
-    """Whether the gfx950 kernel (256 CUs) stores the partials of this plan in fp32: causal plans, and dense plans
-    that split the tiles past a multiple of the CUs rather than those of the last round of resident workgroups.
-    Rows without a plan (a plain bool array) are of the latter kind: fp16."""
-    if causal:
-        return True
-    if getattr(rows, "plan", None) is None:
-        return False
-    n, n_full = rows.plan
-    cus, slots = 256, 256 * {64: 4, 96: 3, 128: 3, 256: 2}[head_dim]
-    kv_tiles, rem, rem_cu = (seq_kv + 63) // 64, n % slots, n % cus
-    ranges = slots // rem if rem else 1
-    if n >= 2 * cus:
-        short_round = ranges >= 4 or (ranges == 3 and (4 * rem <= 3 * cus or kv_tiles >= 112))
-    else:
-        short_round = ranges >= 2 and 2 * rem_cu <= cus
-    if n <= cus or (short_round and kv_tiles >= 48):
-        return False
-    return n - n_full == rem_cu and 2 * rem_cu <= cus   # else two ranges of the last round
+def plan_fp32(workspace: int, n_split: int, chunks: int, layout_dim: int, block_m: int = 128) -> bool:
+    """Whether a plan of the gfx950 kernel (sage_attn_plan) keeps its partials in fp32, by its workspace: per unit (a split
+    tile and one of its ranges) block_m rows of layout_dim values of 2 or 4 bytes and 8 bytes of (m, l)."""
+    size = {4 * layout_dim + 8: True, 2 * layout_dim + 8: False}
+    return size[workspace // (n_split * chunks * block_m)]
 
 
 def round_output(x: np.ndarray, out_dtype: str) -> np.ndarray:

@@ -92,10 +92,11 @@ def fp32_cos_head(q, k, v, out, causal, chunk=4096):
 def kv_split(dev, B, H, Sq, Skv, D, causal, heads=None):
     """The emulation's ``kv_split`` argument that follows the attention kernel's plan on `dev` (None when the plan
     splits nothing).  ``heads``: indices, in the full problem of H heads, of the heads an emulated sample holds."""
-    n_full, chunks, _ = _capi.attn_plan(torch.device(dev).index or 0, B, H, Sq, Skv, D, bool(causal))
+    n_full, chunks, ws = _capi.attn_plan(torch.device(dev).index or 0, B, H, Sq, Skv, D, bool(causal))
     if chunks <= 1:
         return None
-    return chunks, orc.split_rows(B, H, Sq, n_full, heads=heads)
+    fp32 = orc.plan_fp32(ws, B * H * ((Sq + 127) // 128) - n_full, chunks, _capi.layout_dim(D))
+    return chunks, orc.split_rows(B, H, Sq, n_full, heads=heads, fp32=fp32)
 
 
 def unpad(a: np.ndarray, d: int, axis: int = -1) -> np.ndarray:

@@ -777,3 +777,21 @@ def test_seed_binade_holds_the_scores_of_each_head_dim():
     # |S| <= 127^2 * (channels one MFMA sum covers); d96 runs 96 nonzero channels of the 128 layout
     assert orc.seeded(64) and orc.seeded(96) and orc.seeded(128) and not orc.seeded(256)
     assert 127 * 127 * 128 <= 2292099 < 127 * 127 * 256
+
+
+@pytest.mark.parametrize("dl", [64, 128, 256])
+def test_partial_format_follows_the_workspace(dl):
+    """The plan's workspace tells the format of its partials, and the emulation rounds them to fp16 only there."""
+    for fp32, width in ((False, 2), (True, 4)):
+        assert orc.plan_fp32(28 * 8 * 128 * (width * dl + 8), 28, 8, dl) is fp32
+    with pytest.raises(KeyError):
+        orc.plan_fp32(28 * 8 * 128 * (3 * dl + 8), 28, 8, dl)
+    rng = np.random.default_rng(dl)
+    q, k, v = (orc.round_to_bf16(rng.standard_normal((1, 1, s, dl)).astype(np.float32)) for s in (128, 512, 512))
+    q8, qs = orc.quant_q(q)
+    k8, ks, v8, vs = orc.quant_kv(k, v)
+    rows = [orc.split_rows(1, 1, 128, 0, fp32=f) for f in (False, True)]
+    assert [r[:, :, 5:].fp32 for r in rows] == [False, True]
+    half, full = (orc.attention(q8, qs, k8, ks, v8, vs, 512, block_n=32, out_dtype="f32", kv_split=(2, r)) for r in rows)
+    whole = orc.attention(q8, qs, k8, ks, v8, vs, 512, block_n=32, out_dtype="f32")
+    assert 0 < np.abs(full - whole).max() < np.abs(half - whole).max() / 16   # 2^-24 sums against a 2^-11 rounding
