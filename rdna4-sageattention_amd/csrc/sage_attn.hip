@@ -1033,32 +1033,36 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict
 // Work plan.  A launch of n query tiles runs on `cus` CUs, each holding `slots / cus` workgroups (3 at head dims 96 and
 // 128, 4 at 64, 2 at 256); its time follows the CU with the most tiles.  Tiles that would make a short last round
 // have their key range split over `chunks` workgroups (at most 16, at least 4 key tiles each) and a merge kernel
-// combines the parts.  The rules, with attention + merge times in us at L key tiles of 64 (bf16, one MI355X):
-//  * n <= cus: every tile, over slots / n ranges.
-//  * the short last round (n mod slots tiles) leaves at least 3/4 of the slots (n < 2 cus: half) and L >= 48: those
-//    tiles, over slots / (n mod slots) ranges; fp16 partials, the most ranges for the least traffic.  d128, L 72,
-//    n 864 (768 + 96 x 8): 165 against 204 whole; with L < 48 the merge costs more than it gains (d128, L 20, n 288:
-//    42 split, 31 whole; d64, L 14, n 448: 29.5 split, 19.7 whole; d64, L 64, n 1536 over 2 ranges: 176 split, 161
-//    whole).  Three ranges as well where the round has at most 3/4 of a tile per CU (whole calls at d256, n 660,
-//    512 + 148 x 3: L 64 264 against 279 whole, L 512 1754 against 1997) or L >= 112 (n 1024, 768 + 256 x 3: d128
-//    L 64 213 against 205 whole, L 128 385 against 383, L 512 1433 against 1465; d96 L 512 1204 against 1252; d128,
-//    n 10240, L 512 11721 against 11894; d64, n 1344, 1024 + 320 x 3: L 128 298 against 305 with 1280 + 64 x 4).
-//  * else the tiles past the last full multiple of cus, at most cus / 2 of them and L >= 32 (20 past the first
-//    round), over cus / that many ranges: one more unit for every CU instead of one more tile for some.  d64, L 64,
-//    n 640 (512 + 128 x 2): 73 against 86 whole; d128, L 72, n 576: 113 against 122; d128, L 265, n 640: 403 against
-//    442; d256, L 69, n 840 (768 + 72 x 3): 272 against 286; d128, L 72, n 1152 (1024 + 128 x 2): 209 against 218 with
-//    768 + 384 x 2.  Below the line: d128, L 20, n 640: 46 split, 43 whole.  More than cus / 2 tiles: d128, L 72,
-//    n 704: 146 split, 132 whole.
-//  * else two ranges of the last round where L >= 128 and the round leaves CUs without a tile, or without the second
-//    (whole calls): d256, n 768 (512 + 256 x 2), L 96 391 against 388 whole, L 192 716 against 736, L 512 1809 against
-//    1905; d64, n 448, L 64 81 against 78, L 128 136 against 138, L 512 460 against 497; d64, n 1440 (1024 + 416 x 2),
-//    L 256 662 against 672.  Not two full tiles per CU: d64, n 1536, L 512 1307 split, 1275 whole.  fp16 partials.
-//  * causal: every tile of launches of at most cus tiles, the longer the key range the more tiles (L >= n / 4 at 256
-//    CUs).  d128, 192 tiles of a 700-row chunk against 8192 keys (4 ranges): 80 against 120 whole; square 8 x 2048
-//    (128 tiles, L 32): 31 against 35; below the line 16 x 2048 (256 tiles, L 32): 41 split, 36 whole; past one tile
-//    per CU, 384 tiles of 1500 rows against 9001 keys (2 ranges): 152 split, 149 whole, and square 8 x 8192 (512 tiles):
-//    138 split, 126 whole.
-// The tiles of the second and the causal rule keep fp32 partials, the precision they would be accumulated in whole.
+// combines the parts.  Rules for L key tiles of 64, the first that holds (attention + merge in us; bf16, one MI355X, q of
+// N(0, 1), K with a few offset channels; "a / b" = split / whole):
+//  1. n <= cus: every tile, over slots / n ranges.
+//  2. n > cus, the last round (r = n mod slots tiles, over slots / r ranges, fp16 partials):
+//     n < 2 cus, at most cus / 2 tiles past cus: three ranges from L 32 (d64, n 288: L 32 33.0 / 34.1, L 47 40.6 / 47.1,
+//       L 20 28.0 / 23.9), two from L 48 (d128, n 288: L 47 60.6 / 60.5, L 64 73.1 / 78.6).
+//     n >= 2 cus: where its units, one a CU, find every CU free (r * ranges <= cus), from 3 ranges (L 12) or, for r <=
+//       cus / 8, 2 (d128, n 800: L 12 39.5 / 42.9, L 16 46.1 / 52.6; d256, n 544: L 8 46.7 / 48.7, L 16 61.3 / 72.1);
+//       four ranges or more from L 48 (d128, L 72, n 864 = 768 + 96 x 8: 165 / 204), five or more with r > cus / 2 from
+//       L 40 (d128, n 912: L 47 121 / 127, L 32 93 / 91); three from L 48 with r <= 3/4 cus (d256, n 656: L 32 125 / 125,
+//       L 80 257 / 285; whole calls, n 660: L 64 264 / 279, L 512 1754 / 1997), else from L 112 (d128, n 1024: L 64 179 /
+//       171, L 128 385 / 383, L 512 1433 / 1465; d64, n 1344: L 96 212 / 218 by rule 3).
+//  3. The c = n mod cus tiles past the last full multiple of cus, over cus / c ranges, fp32 partials (the precision they
+//     would be accumulated in whole): one more unit for every CU instead of one more tile for some.  n < 2 cus: c <= cus /
+//     4 and L >= 48.  n >= 2 cus: c <= cus / 2, and L >= 20 (d128, n 880: L 20 63 / 63, L 32 86 / 91; d128, n 1376: L 32 119
+//     / 124), or 32 inside the first round (d64, L 64, n 640: 73 / 86; d128, n 640: L 20 47 / 44) and at two workgroups
+//     per CU unless c is a short last round or at most cus / 8 (d256, n 896: L 20 111 / 103, L 32 152 / 149, L 40 183 /
+//     185; n 784, c = 16: L 20 94 / 99).
+//  4. Two ranges of the last round from L 128 where the round leaves CUs without a tile, r <= cus, or without the second,
+//     0 < c <= 3/4 cus; fp16 partials.  d256, n 768: L 80 299 / 295, L 96 350 / 360 (whole calls: L 96 391 / 388, L 192
+//     716 / 736); d64, n 448, L 128 136 / 138; d64, n 1440, L 256 662 / 672.  d64, n 1536 (c = 0), L 512 1307 / 1275.
+//  5. Causal: every tile of launches of at most cus tiles, the longer the key range the more tiles (L >= n / 4 at 256
+//     CUs), fp32 partials.  d128, 192 tiles of a 700-row chunk against 8192 keys (4 ranges): 80 / 120; square 8 x 2048
+//     (128 tiles, L 32): 31 / 35; below the line 16 x 2048 (256 tiles, L 32): 41 / 36; past one tile per CU, 384 tiles of
+//     1500 rows against 9001 keys (2 ranges): 152 / 149, and square 8 x 8192 (512 tiles): 138 / 126.
+// Masked launches plan with the causal flag folded into the mask, rules 1 to 4, less what shorter walks make dearer: rule
+// 2's three ranges below 2 cus from L 48 (d64, n 320, L 40 with 5/8 of the keys, whole call 47 / 42), its units one a CU
+// only where neither the causal flag nor a bool mask's rows shorten some walks (d256, n 576, L 18, causal: 107 / 99), and no
+// rule 3 for bool masks whose rows may see different tiles (a row axis or the causal flag), as their tiles do not end
+// together anyway (a band of 2/3 of the keys, whole calls: d128, n 1312, L 32 157 / 151; d64, n 1568, L 24 117 / 110).
 // ------------------------------------------------------------------------------------------------------------------
 constexpr int CAUSAL_SPLIT_TILES = 256;  // causal launches of more tiles run whole on every device (its CUs at most)
 
@@ -1098,7 +1102,7 @@ static int resident_blocks(int* per_cu) {
 }
 
 template <int HD, bool CAUSAL, int OUT_DT>
-static int make_plan(int B, int H, int Sq, int Skv, AttnPlan* p) {
+static int make_plan(int B, int H, int Sq, int Skv, AttnPlan* p, int walks = WALKS_ALL) {
   constexpr int D = layout_dim(HD);
   const int n = B * H * ((Sq + ATT_BM - 1) / ATT_BM);
   p->n_tiles = n;
@@ -1116,32 +1120,42 @@ static int make_plan(int B, int H, int Sq, int Skv, AttnPlan* p) {
   const int most = min(kv_tiles / 4, ATT_MAX_CHUNKS);
   int rem = 0, chunks = 1;
   if (CAUSAL) {
-    if (n <= cus && (int64_t)kv_tiles * cus >= 64 * (int64_t)n) {
+    if (n <= cus && (int64_t)kv_tiles * cus >= 64 * (int64_t)n) {  // rule 5
       rem = n;
       chunks = min(slots / n, most);
       p->p32 = true;
     }
+  } else if (n <= cus) {  // rule 1
+    rem = n;
+    chunks = min(slots / n, most);
   } else {
-    const int rem_round = n % slots, rem_cu = n % cus;
-    const bool past_one = n >= 2 * cus;  // every CU has at least two tiles
-    const int ranges = rem_round > 0 ? slots / rem_round : 1;
-    const bool round = past_one ? ranges >= 4 || (ranges == 3 && (4 * rem_round <= 3 * cus || kv_tiles >= 112))
-                                : ranges >= 2 && 2 * rem_cu <= cus;
-    if (n <= cus || (round && kv_tiles >= 48)) {
-      rem = rem_round;
-      chunks = rem > 0 ? min(ranges, most) : 1;
-    } else if (rem_cu > 0 && (past_one ? 2 * rem_cu <= cus && kv_tiles >= (n > slots ? 20 : 32)
-                                       : 4 * rem_cu <= cus && kv_tiles >= 48)) {
-      rem = rem_cu;
-      chunks = min(cus / rem, most);
-      p->p32 = true;
-    } else if (ranges >= 2 && kv_tiles >= 128 && (rem_round <= cus || 4 * rem_cu <= 3 * cus) &&
-               (rem_round <= cus || rem_cu > 0)) {
-      rem = rem_round;
+    const int r = n % slots, c = n % cus, L = kv_tiles;
+    const int ranges = r > 0 ? slots / r : 1, units = r * min(ranges, most);
+    bool round, past;
+    if (n < 2 * cus) {
+      round = ranges >= 2 && 2 * c <= cus && L >= (ranges >= 3 && walks == WALKS_ALL ? 32 : 48);
+      past = 4 * c <= cus && L >= 48;
+    } else {
+      round = (walks <= WALKS_MASKED && units <= cus && min(ranges, most) >= (8 * r <= cus ? 2 : 3)) ||
+              (ranges >= 4 && L >= (ranges >= 5 && 2 * r > cus ? 40 : 48)) ||
+              (ranges == 3 && L >= (4 * r <= 3 * cus ? 48 : 112));
+      past = 2 * c <= cus && L >= (n < slots || (per_cu <= 2 && c != r && 8 * c > cus) ? 32 : 20);
+    }
+    past = past && c > 0 && walks != WALKS_DIFFER;
+    const bool two = ranges >= 2 && L >= 128 && (r <= cus || (c > 0 && 4 * c <= 3 * cus));
+    if (round || (two && !past)) {  // rules 2 and 4
+      rem = r;
       chunks = min(ranges, most);
+    } else if (past) {  // rule 3
+      rem = c;
+      chunks = min(cus / c, most);
+      p->p32 = true;
     }
   }
-  if (chunks < 2) return SAGE_OK;
+  if (chunks < 2) {
+    p->p32 = false;
+    return SAGE_OK;
+  }
   p->n_full = n - rem;
   p->chunks = chunks;
   p->workspace = ws_bytes((int64_t)rem * chunks, D, p->p32);
@@ -1286,16 +1300,15 @@ int attn_varlen_impl(const int8_t* q8, const float* qs, const int8_t* k8, const 
 }
 
 // Masked attention (the mask variant of the kernel; validation by the caller, sage_forward_masked).  The plan is
-// the dense non-causal one (sage_attn_plan with causal = 0; the causal flag lives in the mask bits), so callers can
-// query it; the mask variant's occupancy is never below the dense kernel's.
+// the non-causal one (the causal flag lives in the mask bits) for the mask's walks.  The mask variant's occupancy is never below the dense kernel's.
 template <int HD, bool CAUSAL, int OUT_DT>
-static int plan_mask(int B, int H, int Sq, int Skv, AttnPlan* p) {
-  return make_plan<HD, false, OUT_DT>(B, H, Sq, Skv, p);
+static int plan_mask(int B, int H, int Sq, int Skv, int walks, AttnPlan* p) {
+  return make_plan<HD, false, OUT_DT>(B, H, Sq, Skv, p, walks);
 }
 
-int attn_mask_plan_impl(int B, int H, int Sq, int Skv, int D, int64_t* ws) {
+int attn_mask_plan_impl(int B, int H, int Sq, int Skv, int D, int walks, int64_t* ws) {
   AttnPlan p;
-  int rc = SAGE_ATTN_DISPATCH(D, false, true, plan_mask, B, H, Sq, Skv, &p);
+  int rc = SAGE_ATTN_DISPATCH(D, false, true, plan_mask, B, H, Sq, Skv, walks, &p);
   if (rc) return rc;
   *ws = p.workspace;
   return SAGE_OK;
@@ -1304,11 +1317,11 @@ int attn_mask_plan_impl(int B, int H, int Sq, int Skv, int D, int64_t* ws) {
 template <int HD, bool ADDITIVE, int OUT_DT>
 static int launch_attn_mask(const int8_t* q8, const float* qs, const int8_t* k8, const float* ks, const uint8_t* v8t,
                             const float* vs, void* out, int64_t osb, int64_t oss, int64_t osh, int B, int H, int Hkv,
-                            int Sq, int Skv, int hd, MaskTabs mt, void* workspace, hipStream_t st) {
+                            int Sq, int Skv, int hd, MaskTabs mt, int walks, void* workspace, hipStream_t st) {
   constexpr int D = layout_dim(HD);
   AttnPlan p;
   int rc;
-  if ((rc = plan_mask<HD, false, OUT_DT>(B, H, Sq, Skv, &p))) return rc;
+  if ((rc = plan_mask<HD, false, OUT_DT>(B, H, Sq, Skv, walks, &p))) return rc;
   const int q_tiles = (Sq + ATT_BM - 1) / ATT_BM;
   const int n_split = p.n_tiles - p.n_full;
   const int blocks = p.n_full + n_split * p.chunks;
@@ -1329,9 +1342,9 @@ static int launch_attn_mask(const int8_t* q8, const float* qs, const int8_t* k8,
 // workspace: at least attn_mask_plan_impl bytes (may be NULL when that is 0)
 int attn_mask_impl(const int8_t* q8, const float* qs, const int8_t* k8, const float* ks, const uint8_t* v8t,
                    const float* vs, void* out, int64_t osb, int64_t oss, int64_t osh, int B, int H, int Hkv, int Sq,
-                   int Skv, int D, int out_dtype, const MaskTabs* mt, void* workspace, void* stream) {
+                   int Skv, int D, int out_dtype, const MaskTabs* mt, int walks, void* workspace, void* stream) {
   return SAGE_ATTN_DISPATCH(D, mt->raw != nullptr, out_dtype == SAGE_DTYPE_BF16, launch_attn_mask, q8, qs, k8, ks, v8t, vs, out,
-                            osb, oss, osh, B, H, Hkv, Sq, Skv, D, *mt, workspace, (hipStream_t)stream);
+                            osb, oss, osh, B, H, Hkv, Sq, Skv, D, *mt, walks, workspace, (hipStream_t)stream);
 }
 
 }  // namespace sage

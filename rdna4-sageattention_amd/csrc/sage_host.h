@@ -50,6 +50,10 @@ __host__ __device__ constexpr int layout_dim(int d) { return d == 96 ? 128 : d; 
 // padded KV length used by every K8 / KS / V8T layout
 inline int kv_pad(int skv) { return (skv + SAGE_KV_PAD - 1) / SAGE_KV_PAD * SAGE_KV_PAD; }
 
+// What the attention plan knows of the tiles' walks: over every key (no mask), over those a mask leaves, over those an
+// additive mask and the causal flag leave, or over those a bool mask leaves to each row block (a row axis, or causal).
+constexpr int WALKS_ALL = 0, WALKS_MASKED = 1, WALKS_CAUSAL_BIAS = 2, WALKS_DIFFER = 3;
+
 // Boolean attention mask as the attention kernel reads it (built by mask_prep_block and mask_range_block of
 // sage_mask.h, inside the two quantization launches).
 // bits: one 32-bit word per (row, 64-key tile, lane half hf): bit 16 kb + v is the visibility of the key that the QK

@@ -24,10 +24,10 @@ int forward_quant_impl(const void*, int64_t, int64_t, int64_t, const void*, int6
                        int64_t, int64_t, int64_t, int, int, int, int, int, int, int, float, int8_t*, float*, float*,
                        int8_t*, float*, uint8_t*, float*, const MaskPrep*, void*);
 int64_t vamax_partial_bytes(int B, int Hkv, int Skv, int D);
-int attn_mask_plan_impl(int B, int H, int Sq, int Skv, int D, int64_t* ws);
+int attn_mask_plan_impl(int B, int H, int Sq, int Skv, int D, int walks, int64_t* ws);
 int attn_mask_impl(const int8_t* q8, const float* qs, const int8_t* k8, const float* ks, const uint8_t* v8t,
                    const float* vs, void* out, int64_t osb, int64_t oss, int64_t osh, int B, int H, int Hkv, int Sq,
-                   int Skv, int D, int out_dtype, const MaskTabs* mt, void* workspace, void* stream);
+                   int Skv, int D, int out_dtype, const MaskTabs* mt, int walks, void* workspace, void* stream);
 
 // Extents of the tables.  A mask axis with stride 0 (broadcast) is stored once; rows are stored when the mask has a
 // row axis or the causal flag makes rows differ.
@@ -54,6 +54,11 @@ static MaskShape mask_shape(int B, int H, int Sq, int Skv, int64_t msb, int64_t 
   return m;
 }
 
+static int mask_walks(const MaskShape& m, int causal) {
+  if (m.additive) return causal ? WALKS_CAUSAL_BIAS : WALKS_MASKED;
+  return m.mq > 1 ? WALKS_DIFFER : WALKS_MASKED;
+}
+
 static int64_t align256(int64_t n) { return (n + 255) / 256 * 256; }
 
 // Workspace of sage_forward_masked: the attention plan's split state, the per-chunk V maxima, the bits, the classes,
@@ -62,8 +67,9 @@ struct MaskWorkspace {
   int64_t attn, vpart, bits, cls, range, bias, total;
 };
 
-static int mask_workspace(int B, int H, int Hkv, int Sq, int Skv, int D, const MaskShape& m, MaskWorkspace* w) {
-  int rc = attn_mask_plan_impl(B, H, Sq, Skv, D, &w->attn);
+static int mask_workspace(int B, int H, int Hkv, int Sq, int Skv, int D, int causal, const MaskShape& m,
+                          MaskWorkspace* w) {
+  int rc = attn_mask_plan_impl(B, H, Sq, Skv, D, mask_walks(m, causal), &w->attn);
   if (rc) return rc;
   w->vpart = align256(w->attn);
   w->bits = w->vpart + align256(vamax_partial_bytes(B, Hkv, Skv, D));
@@ -108,7 +114,7 @@ int sage_mask_workspace(int B, int H, int Hkv, int Sq, int Skv, int D, int causa
   if (rc) return rc;
   const sage::MaskShape m = sage::mask_shape(B, H, Sq, Skv, msb, msh, msq, causal, mask_dtype);
   sage::MaskWorkspace w;
-  if ((rc = sage::mask_workspace(B, H, Hkv, Sq, Skv, D, m, &w))) return rc;
+  if ((rc = sage::mask_workspace(B, H, Hkv, Sq, Skv, D, causal, m, &w))) return rc;
   *workspace_bytes = w.total;
   return SAGE_OK;
 }
@@ -137,7 +143,7 @@ int sage_forward_masked(const void* q, int64_t qsb, int64_t qss, int64_t qsh, co
                "%s: workspace must be non-NULL and 256-byte aligned", who);
   const sage::MaskShape m = sage::mask_shape(B, H, Sq, Skv, msb, msh, msq, causal, mask_dtype);
   sage::MaskWorkspace w;
-  if ((rc = sage::mask_workspace(B, H, Hkv, Sq, Skv, D, m, &w))) return rc;
+  if ((rc = sage::mask_workspace(B, H, Hkv, Sq, Skv, D, causal, m, &w))) return rc;
   SAGE_REQUIRE(workspace_bytes >= w.total, "%s: workspace of %lld bytes, the call needs %lld", who,
                (long long)workspace_bytes, (long long)w.total);
   // q / k / v and the intermediates are checked by the quantization step before it launches anything
@@ -195,7 +201,7 @@ int sage_forward_masked(const void* q, int64_t qsb, int64_t qss, int64_t qsh, co
                           m.mg,
                           m.nrb};
   return sage::attn_mask_impl(q8, qs, k8, ks, v8t, vs, out, osb, oss, osh, B, H, Hkv, Sq, Skv, D, dtype, &mt,
-                              w.attn ? workspace : nullptr, stream);
+                              sage::mask_walks(m, causal), w.attn ? workspace : nullptr, stream);
 }
 
 }  // extern "C"

@@ -147,3 +147,21 @@ def test_three_ranges_of_head_dim_256_against_whole_tiles(dev):
     whole, split = outs
     # the same probabilities: the fp16 partials' rounding (2^-11) and the output's own (2^-9, twice)
     assert (split - whole).norm() <= 2.0 ** -8 * whole.norm()
+
+
+@pytest.mark.parametrize("B,H,Sq,L,D,n_full,chunks,fp32", [
+    (1, 16, 2304, 31, 64, 288, 1, False), (1, 16, 2304, 32, 64, 0, 3, False),     # up to half a tile per CU past the first
+    (1, 16, 2944, 47, 64, 368, 1, False), (1, 16, 2944, 48, 64, 0, 2, False),
+    (1, 16, 6400, 7, 128, 800, 1, False), (1, 16, 6400, 8, 128, 768, 2, False),   # 32 tiles past a full round
+    (1, 16, 6656, 11, 128, 832, 1, False), (1, 16, 6656, 12, 128, 768, 3, False),  # 64: from three ranges, one unit a CU
+    (1, 16, 6656, 19, 96, 768, 4, False), (1, 16, 6656, 20, 96, 768, 4, True),     # five would not fit: past the CUs, fp32
+    (1, 16, 7296, 39, 128, 912, 1, False), (1, 16, 7296, 40, 128, 768, 5, False),  # more than half a tile per CU
+    (1, 16, 4352, 16, 256, 512, 4, False), (1, 16, 4352, 20, 256, 512, 5, False),
+    (1, 16, 7168, 31, 256, 896, 1, False), (1, 16, 7168, 32, 256, 768, 2, True),   # two workgroups per CU
+    (1, 16, 6272, 20, 256, 768, 5, True),
+])
+def test_plan_of_short_walks(dev, B, H, Sq, L, D, n_full, chunks, fp32):
+    full, ch, ws = _capi.attn_plan(dev.index or 0, B, H, Sq, L * 64, D, 0)
+    assert (full, ch) == (n_full, chunks)
+    rem, dl = B * H * ((Sq + 127) // 128) - full, _capi.layout_dim(D)
+    assert ws == (rem * ch * 128 * ((4 if fp32 else 2) * dl + 8) if ch > 1 else 0)
