@@ -183,6 +183,18 @@ int sage_forward_varlen(const void* q, int64_t qss, int64_t qsh, const void* k, 
                         float* ks, uint8_t* v8t, float* vs, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * sage_forward_varlen of the sequences with at least min_kv keys, heads * queries * keys (halved, rounded down, when
+ * causal) >= min_work and, when causal, no more queries than keys: the sequences that the reference's router sends to
+ * its kernel (src/rdna4_sage/__init__.py:61-69, per sequence).  The output rows of the others are not written.
+ */
+int sage_forward_varlen_routed(const void* q, int64_t qss, int64_t qsh, const void* k, int64_t kss, int64_t ksh,
+                               const void* v, int64_t vss, int64_t vsh, void* out, int64_t oss, int64_t osh,
+                               const int* cu_seqlens_q, const int* cu_seqlens_k, int batch, int H, int Hkv, int total_q,
+                               int total_k, int D, int dtype, int causal, float qs_mul, int64_t min_kv, int64_t min_work,
+                               int8_t* q8, float* qs, int8_t* k8, float* ks, uint8_t* v8t, float* vs, void* workspace,
+                               int64_t workspace_bytes, void* stream);
+
+/*
  * Attention masks with torch SDPA's semantics: mask_dtype SAGE_DTYPE_BOOL (a nonzero byte = the query attends the
  * key) or an additive float mask of the inputs' dtype (SAGE_DTYPE_BF16 / SAGE_DTYPE_F16: added to the scaled scores,
  * -inf = masked).  The mask is addressed as mask + b*msb + h*msh + i*msq + j (in elements) for batch b, query head h,

@@ -23,6 +23,7 @@ LSE_HEAD_DIMS = tuple(_MANIFEST["lse"]["head_dims"])   # head dims of the public
 ARCHS = (_MANIFEST["arch"],)
 DTYPES = {torch.bfloat16: _capi.DTYPE_BF16, torch.float16: _capi.DTYPE_F16}
 _I32_MAX = 2**31 - 1
+_I64_MIN, _I64_MAX = -2**63, 2**63 - 1
 
 _arch_cache = {}
 
@@ -261,6 +262,13 @@ def attention_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q=None, max
     are 0.  Rows outside every sequence are left unwritten (as torch.empty_like).  Returns [total_q, H, D].
     The reference loops over the sequences on the host (src/sageattention/core.py:80-88).  Invalid cu_seqlens
     (decreasing or past the totals) leave the output unwritten instead of raising, since they are not read back."""
+    return packed_pass(q, k, v, cu_seqlens_q, cu_seqlens_k, sm_scale, is_causal)
+
+
+def packed_pass(q, k, v, cu_seqlens_q, cu_seqlens_k, sm_scale=None, is_causal=False, route=None):
+    """attention_varlen; with route = (min_kv, min_work) only of the sequences with at least min_kv keys and a work (heads *
+    q_len * kv_len, halved when causal) of at least min_work, causal ones with q_len <= kv_len.  The rows of the others are
+    left unwritten: each costs a few empty workgroups, and no more where the route takes no sequence at all."""
     if not (q.is_cuda and k.device == q.device and v.device == q.device):
         raise Unsupported("tensors must be on one ROCm GPU")
     if q.dtype not in DTYPES or k.dtype != q.dtype or v.dtype != q.dtype:
@@ -290,10 +298,11 @@ def attention_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q=None, max
     q8, qs, k8, ks, v8t, vs, ws = (buf.data_ptr() + o for o in offs)
     out = torch.empty((TQ, H, D), device=dev, dtype=q.dtype)
     with torch.cuda.device(dev):
-        _capi.call("sage_forward_varlen", _ptr(q), *sq_, _ptr(k), *sk_, _ptr(v), *sv_, _ptr(out), out.stride(0),
-                   out.stride(1), _ptr(cu_q), _ptr(cu_k), batch, H, Hkv, TQ, TK, D, DTYPES[q.dtype],
-                   int(bool(is_causal)), qs_fold_factor(sm_scale, D), q8, qs, k8, ks, v8t, vs, ws, ws_bytes,
-                   torch.cuda.current_stream(dev).cuda_stream)
+        _capi.call("sage_forward_varlen" if route is None else "sage_forward_varlen_routed", _ptr(q), *sq_, _ptr(k), *sk_,
+                   _ptr(v), *sv_, _ptr(out), out.stride(0), out.stride(1), _ptr(cu_q), _ptr(cu_k), batch, H, Hkv, TQ, TK, D,
+                   DTYPES[q.dtype], int(bool(is_causal)), qs_fold_factor(sm_scale, D),
+                   *(() if route is None else (max(_I64_MIN, min(_I64_MAX, x)) for x in route)),
+                   q8, qs, k8, ks, v8t, vs, ws, ws_bytes, torch.cuda.current_stream(dev).cuda_stream)
     return out
 
 

@@ -48,6 +48,8 @@ SIGNATURES = {
     "sage_varlen_layout": ([_I, _I, _I, _I, _I, _P, _P], _I),
     "sage_forward_varlen": ([_P, _L, _L, _P, _L, _L, _P, _L, _L, _P, _L, _L, _P, _P,
                              _I, _I, _I, _I, _I, _I, _I, _I, _F, _P, _P, _P, _P, _P, _P, _P, _L, _P], _I),
+    "sage_forward_varlen_routed": ([_P, _L, _L, _P, _L, _L, _P, _L, _L, _P, _L, _L, _P, _P,
+                                    _I, _I, _I, _I, _I, _I, _I, _I, _F, _L, _L, _P, _P, _P, _P, _P, _P, _P, _L, _P], _I),
     "sage_mask_workspace": ([_I, _I, _I, _I, _I, _I, _I, _I, _L, _L, _L, _P], _I),
     "sage_forward_masked": ([_P, _L, _L, _L, _P, _L, _L, _L, _P, _L, _L, _L, _P, _L, _L, _L,
                              _I, _I, _I, _I, _I, _I, _I, _I, _F, _P, _I, _L, _L, _L,

@@ -593,6 +593,7 @@ struct VarlenKeys {
   const int* cu_k;  // [batch + 1] token offsets of the sequences in k / v
   const int* kp;    // [batch + 1] padded row offsets
   const int* ktab;  // [TKP / 128] owner of each padded 128-key block
+  const int* hdr;   // [1]: query tiles of the batch
 };
 
 // first launch: blocks [0, nv) per-channel V maxima of one padded 128-key block (atomicMax into vs), [nv, nv + nk)
@@ -625,7 +626,7 @@ __global__ __launch_bounds__(256) void quant_varlen_kernel(const uint16_t* __res
     const int kb = vk.cu_k[seq];
     quant_k64_core<D, DT>(k + h * ksh + (int64_t)kb * kss, kss, g * 64 - vk.kp[seq], vk.cu_k[seq + 1] - kb,
                           k8 + ((int64_t)h * TKP + g * 64) * HeadDim<D>::DP, ks + (int64_t)h * (TKP / SAGE_KV_BLOCK) + g * 2);
-  } else {
+  } else if (vk.hdr[1] > 0) {  // (no tile, no Q: a routed batch without a sequence for this pass)
     quant_q_rows<D, DT>(x, 0, qss, qsh, H, TQ, row_tiles, qs_mul, q8, qs, blk - nv - nk);
   }
 }
@@ -825,9 +826,9 @@ int forward_quant_impl(const void* q, int64_t qsb, int64_t qss, int64_t qsh, con
 // Validation is done by the caller (sage_forward_varlen); vs must already be zero.
 int varlen_quant_impl(const void* q, int64_t qss, int64_t qsh, const void* k, int64_t kss, int64_t ksh, const void* v,
                       int64_t vss, int64_t vsh, int H, int Hkv, int TQ, int TKP, int D, int dtype, float qs_mul,
-                      const int* cu_k, const int* kp, const int* ktab, int8_t* q8, float* qs, int8_t* k8, float* ks,
-                      uint8_t* v8t, float* vs, void* stream) {
-  const VarlenKeys vk{cu_k, kp, ktab};
+                      const int* cu_k, const int* kp, const int* ktab, const int* hdr, int8_t* q8, float* qs, int8_t* k8,
+                      float* ks, uint8_t* v8t, float* vs, void* stream) {
+  const VarlenKeys vk{cu_k, kp, ktab, hdr};
   SAGE_DISPATCH_D_DT(D, dtype, launch_varlen_quant, q, qss, qsh, k, kss, ksh, v, vss, vsh, H, Hkv, TQ, TKP, qs_mul, vk,
                      q8, qs, k8, ks, v8t, vs, (hipStream_t)stream);
   return check_launch("varlen quantization launch");

@@ -24,8 +24,8 @@ namespace sage {
 
 int varlen_quant_impl(const void* q, int64_t qss, int64_t qsh, const void* k, int64_t kss, int64_t ksh, const void* v,
                       int64_t vss, int64_t vsh, int H, int Hkv, int TQ, int TKP, int D, int dtype, float qs_mul,
-                      const int* cu_k, const int* kp, const int* ktab, int8_t* q8, float* qs, int8_t* k8, float* ks,
-                      uint8_t* v8t, float* vs, void* stream);
+                      const int* cu_k, const int* kp, const int* ktab, const int* hdr, int8_t* q8, float* qs, int8_t* k8,
+                      float* ks, uint8_t* v8t, float* vs, void* stream);
 int attn_varlen_impl(const int8_t* q8, const float* qs, const int8_t* k8, const float* ks, const uint8_t* v8t,
                      const float* vs, void* out, int64_t oss, int64_t osh, int H, int Hkv, int TQ, int TKP, int D,
                      int causal, int out_dtype, int n_blocks, const void* tiles, const int* cu_q, const int* cu_k,
@@ -104,9 +104,27 @@ __device__ __forceinline__ int wave_inclusive_scan(int x) {
 
 __device__ __forceinline__ int pad128(int n) { return (n + 127) / 128 * 128; }
 
+// Which sequences the pass takes (sage_forward_varlen_routed): the others have no query tile and no key block, so that
+// every later launch passes them by; sage_forward_varlen takes all.
+struct VarlenRoute {
+  bool all;
+  int64_t min_kv, min_work;
+};
+
+// Lengths (queries, keys) of sequence b as the pass sees it.
+__device__ __forceinline__ int2 varlen_lengths(const int* cu_q, const int* cu_k, int b, int H, int causal,
+                                               const VarlenRoute& route) {
+  const int sq = cu_q[b + 1] - cu_q[b], sk = cu_k[b + 1] - cu_k[b];
+  if (route.all) return make_int2(sq, sk);
+  const int64_t work = (int64_t)H * sq * sk;
+  const bool takes = sk >= route.min_kv && (causal ? work / 2 : work) >= route.min_work && !(causal && sq > sk);
+  return takes ? make_int2(sq, sk) : make_int2(0, 0);
+}
+
 __global__ __launch_bounds__(VL_META_THREADS) void varlen_meta_kernel(const int* __restrict__ cu_q,
                                                                        const int* __restrict__ cu_k, int batch, int H,
-                                                                       int total_q, int total_k, int* __restrict__ hdr,
+                                                                       int total_q, int total_k, int causal,
+                                                                       VarlenRoute route, int* __restrict__ hdr,
                                                                        int* __restrict__ kp, int* __restrict__ order,
                                                                        int* __restrict__ tpre) {
   __shared__ int buf[VL_META_THREADS];
@@ -124,7 +142,7 @@ __global__ __launch_bounds__(VL_META_THREADS) void varlen_meta_kernel(const int*
   for (int b = lo; b < hi; ++b) {
     const int q0 = cu_q[b], q1 = cu_q[b + 1], k0 = cu_k[b], k1 = cu_k[b + 1];
     if (q0 < 0 || q1 < q0 || q1 > total_q || k0 < 0 || k1 < k0 || k1 > total_k) bad = 1;
-    sk += pad128(k1 - k0);
+    sk += pad128(varlen_lengths(cu_q, cu_k, b, H, causal, route).y);
   }
   __syncthreads();
   if (bad) {  // uniform: every table stays empty
@@ -139,13 +157,13 @@ __global__ __launch_bounds__(VL_META_THREADS) void varlen_meta_kernel(const int*
   int run = block_inclusive_scan(sk, buf) - sk;
   for (int b = lo; b < hi; ++b) {
     kp[b] = run;
-    run += pad128(cu_k[b + 1] - cu_k[b]);
+    run += pad128(varlen_lengths(cu_q, cu_k, b, H, causal, route).y);
   }
   if (t == VL_META_THREADS - 1) kp[batch] = run;  // the last thread's running sum is the total
 
   // ---- order: counting sort by key tiles, descending (positions inside a bin follow LDS atomics) ----
   for (int b = lo; b < hi; ++b) {
-    const int key = min((cu_k[b + 1] - cu_k[b] + 63) / 64, VL_SORT_BINS - 1);
+    const int key = min((varlen_lengths(cu_q, cu_k, b, H, causal, route).y + 63) / 64, VL_SORT_BINS - 1);
     atomicAdd(&bins[VL_SORT_BINS - 1 - key], 1);
   }
   __syncthreads();
@@ -166,7 +184,7 @@ __global__ __launch_bounds__(VL_META_THREADS) void varlen_meta_kernel(const int*
   }
   __syncthreads();
   for (int b = lo; b < hi; ++b) {
-    const int key = min((cu_k[b + 1] - cu_k[b] + 63) / 64, VL_SORT_BINS - 1);
+    const int key = min((varlen_lengths(cu_q, cu_k, b, H, causal, route).y + 63) / 64, VL_SORT_BINS - 1);
     order[atomicAdd(&bins[VL_SORT_BINS - 1 - key], 1)] = b;
   }
   __syncthreads();  // order[] (global, written by this workgroup) is visible to the workgroup after the barrier
@@ -174,14 +192,12 @@ __global__ __launch_bounds__(VL_META_THREADS) void varlen_meta_kernel(const int*
   // ---- tpre: exclusive prefix of H * query tiles over the sorted order ----
   int st = 0;
   for (int i = lo; i < hi; ++i) {
-    const int b = order[i];
-    st += H * ((cu_q[b + 1] - cu_q[b] + 127) / 128);
+    st += H * ((varlen_lengths(cu_q, cu_k, order[i], H, causal, route).x + 127) / 128);
   }
   run = block_inclusive_scan(st, buf) - st;
   for (int i = lo; i < hi; ++i) {
     tpre[i] = run;
-    const int b = order[i];
-    run += H * ((cu_q[b + 1] - cu_q[b] + 127) / 128);
+    run += H * ((varlen_lengths(cu_q, cu_k, order[i], H, causal, route).x + 127) / 128);
   }
   if (t == VL_META_THREADS - 1) {
     tpre[batch] = run;
@@ -265,28 +281,31 @@ __global__ __launch_bounds__(256) void varlen_prep_kernel(const int* __restrict_
 // 640 to 4608 509 -> 506; 60 of 1100, 8 heads x 64, 222 -> 220.
 __global__ __launch_bounds__(256) void varlen_tables_kernel(const int* __restrict__ cu_q, const int* __restrict__ cu_k,
                                                             int batch, int H, int total_q, int total_k, int causal,
-                                                            int* __restrict__ hdr, int* __restrict__ kp_out, int n_tiles,
+                                                            VarlenRoute route, int* __restrict__ hdr,
+                                                            int* __restrict__ kp_out, int n_tiles,
                                                             int n_kblk, int4* __restrict__ tiles, int* __restrict__ ktab,
                                                             float* __restrict__ vs, int64_t n_vs) {
   __shared__ int kp[VL_WAVE + 1], tpre[VL_WAVE + 1], order[VL_WAVE], nq[VL_WAVE], bad;
   const int t = threadIdx.x;
   if (t < VL_WAVE) {
     int q0 = 0, q1 = 0, k0 = 0, k1 = 0;
+    int2 len = make_int2(0, 0);
     if (t < batch) {
       q0 = cu_q[t];
       q1 = cu_q[t + 1];
       k0 = cu_k[t];
       k1 = cu_k[t + 1];
+      len = varlen_lengths(cu_q, cu_k, t, H, causal, route);
     }
     const bool wrong = q0 < 0 || q1 < q0 || q1 > total_q || k0 < 0 || k1 < k0 || k1 > total_k;
     const uint64_t any_wrong = __ballot(wrong);
-    if (any_wrong) q0 = q1 = k0 = k1 = 0;  // every table stays empty
+    if (any_wrong) len = make_int2(0, 0);  // every table stays empty
     if (t == 0) {
       bad = any_wrong != 0;
       kp[0] = tpre[0] = 0;
     }
-    kp[t + 1] = wave_inclusive_scan(pad128(k1 - k0));
-    const int key = t < batch ? (k1 - k0 + 63) / 64 : -1;  // lanes without a sequence rank last
+    kp[t + 1] = wave_inclusive_scan(pad128(len.y));
+    const int key = t < batch ? (len.y + 63) / 64 : -1;  // lanes without a sequence rank last
     int rank = 0;
 #pragma unroll
     for (int j = 0; j < VL_WAVE; ++j) {
@@ -294,7 +313,7 @@ __global__ __launch_bounds__(256) void varlen_tables_kernel(const int* __restric
       rank += kj > key || (kj == key && j < t);
     }
     order[rank] = t;
-    nq[rank] = (q1 - q0 + 127) / 128;
+    nq[rank] = (len.x + 127) / 128;
   }
   __syncthreads();
   if (t < VL_WAVE) tpre[t + 1] = wave_inclusive_scan(H * nq[t]);
@@ -319,6 +338,63 @@ static int check_packed(const void* p, int64_t ss, int64_t sh, const char* name)
   return SAGE_OK;
 }
 
+// sage_forward_varlen of the sequences that `route` takes
+static int forward_varlen(const void* q, int64_t qss, int64_t qsh, const void* k, int64_t kss, int64_t ksh, const void* v,
+                          int64_t vss, int64_t vsh, void* out, int64_t oss, int64_t osh, const int* cu_seqlens_q,
+                          const int* cu_seqlens_k, int batch, int H, int Hkv, int total_q, int total_k, int D, int dtype,
+                          int causal, float qs_mul, VarlenRoute route, int8_t* q8, float* qs, int8_t* k8, float* ks,
+                          uint8_t* v8t, float* vs, void* workspace, int64_t workspace_bytes, void* stream) {
+  VarlenLayout L;
+  int rc = varlen_layout(batch, H, Hkv, total_q, total_k, &L);
+  if (rc) return rc;
+  if (!head_dim_ok(D))
+    return fail(SAGE_ERR_UNSUPPORTED, "sage_forward_varlen: head_dim %d (supported 64, 96, 128, 256)", D);
+  if (dtype != SAGE_DTYPE_BF16 && dtype != SAGE_DTYPE_F16)
+    return fail(SAGE_ERR_UNSUPPORTED, "sage_forward_varlen: dtype code %d (bf16=0, f16=1)", dtype);
+  if ((rc = check_packed(q, qss, qsh, "q"))) return rc;
+  if ((rc = check_packed(k, kss, ksh, "k"))) return rc;
+  if ((rc = check_packed(v, vss, vsh, "v"))) return rc;
+  if ((rc = check_packed(out, oss, osh, "out"))) return rc;
+  if ((rc = check_qs_mul(qs_mul, "sage_forward_varlen"))) return rc;
+  SAGE_REQUIRE(cu_seqlens_q && cu_seqlens_k, "sage_forward_varlen: cu_seqlens is NULL");
+  SAGE_REQUIRE(q8 && qs && k8 && ks && v8t && vs, "sage_forward_varlen: an intermediate pointer is NULL");
+  SAGE_REQUIRE(aligned16(q8) && aligned16(k8) && aligned16(v8t) && aligned16(vs),
+               "sage_forward_varlen: q8 / k8 / v8t / vs must be 16-byte aligned");
+  SAGE_REQUIRE(workspace != nullptr && workspace_bytes >= L.bytes,
+               "sage_forward_varlen: workspace of %lld bytes, the layout needs %lld", (long long)workspace_bytes,
+               (long long)L.bytes);
+  SAGE_REQUIRE(((uintptr_t)workspace & 255u) == 0, "sage_forward_varlen: workspace must be 256-byte aligned");
+  char* ws = static_cast<char*>(workspace);
+  int* hdr = reinterpret_cast<int*>(ws + L.hdr);
+  int* kp = reinterpret_cast<int*>(ws + L.kp);
+  int* order = reinterpret_cast<int*>(ws + L.order);
+  int* tpre = reinterpret_cast<int*>(ws + L.tpre);
+  int* ktab = reinterpret_cast<int*>(ws + L.ktab);
+  int4* tiles = reinterpret_cast<int4*>(ws + L.tiles);
+  hipStream_t st = (hipStream_t)stream;
+
+  const int n_kblk = L.tkp / 128;
+  const int64_t n_vs = (int64_t)batch * Hkv * layout_dim(D);
+  const int64_t n_items = std::max<int64_t>(std::max(L.n_blocks, n_kblk), n_vs);
+  const int grid = (int)std::min<int64_t>((n_items + 255) / 256, 4096);
+  if (batch <= VL_WAVE) {
+    hipLaunchKernelGGL(varlen_tables_kernel, dim3(grid), dim3(256), 0, st, cu_seqlens_q, cu_seqlens_k, batch, H,
+                       total_q, total_k, causal ? 1 : 0, route, hdr, kp, L.n_blocks, n_kblk, tiles, ktab, vs, n_vs);
+  } else {
+    hipLaunchKernelGGL(varlen_meta_kernel, dim3(1), dim3(VL_META_THREADS), 0, st, cu_seqlens_q,
+                       cu_seqlens_k, batch, H, total_q, total_k, causal ? 1 : 0, route, hdr, kp, order, tpre);
+    if ((rc = check_launch("varlen meta launch"))) return rc;
+    hipLaunchKernelGGL(varlen_prep_kernel, dim3(grid), dim3(256), 0, st, hdr, cu_seqlens_q, kp, order, tpre, batch,
+                       H, causal ? 1 : 0, L.n_blocks, n_kblk, tiles, ktab, vs, n_vs);
+  }
+  if ((rc = check_launch("varlen table launch"))) return rc;
+  if ((rc = varlen_quant_impl(q, qss, qsh, k, kss, ksh, v, vss, vsh, H, Hkv, total_q, L.tkp, D, dtype, qs_mul,
+                                    cu_seqlens_k, kp, ktab, hdr, q8, qs, k8, ks, v8t, vs, stream)))
+    return rc;
+  return attn_varlen_impl(q8, qs, k8, ks, v8t, vs, out, oss, osh, H, Hkv, total_q, L.tkp, D, causal, dtype,
+                                L.n_blocks, tiles, cu_seqlens_q, cu_seqlens_k, kp, stream);
+}
+
 }  // namespace sage
 
 extern "C" {
@@ -339,55 +415,21 @@ int sage_forward_varlen(const void* q, int64_t qss, int64_t qsh, const void* k, 
                         int total_k, int D, int dtype, int causal, float qs_mul, int8_t* q8, float* qs, int8_t* k8,
                         float* ks, uint8_t* v8t, float* vs, void* workspace, int64_t workspace_bytes, void* stream) {
   sage::clear_error();
-  sage::VarlenLayout L;
-  int rc = sage::varlen_layout(batch, H, Hkv, total_q, total_k, &L);
-  if (rc) return rc;
-  if (!sage::head_dim_ok(D))
-    return sage::fail(SAGE_ERR_UNSUPPORTED, "sage_forward_varlen: head_dim %d (supported 64, 96, 128, 256)", D);
-  if (dtype != SAGE_DTYPE_BF16 && dtype != SAGE_DTYPE_F16)
-    return sage::fail(SAGE_ERR_UNSUPPORTED, "sage_forward_varlen: dtype code %d (bf16=0, f16=1)", dtype);
-  if ((rc = sage::check_packed(q, qss, qsh, "q"))) return rc;
-  if ((rc = sage::check_packed(k, kss, ksh, "k"))) return rc;
-  if ((rc = sage::check_packed(v, vss, vsh, "v"))) return rc;
-  if ((rc = sage::check_packed(out, oss, osh, "out"))) return rc;
-  if ((rc = sage::check_qs_mul(qs_mul, "sage_forward_varlen"))) return rc;
-  SAGE_REQUIRE(cu_seqlens_q && cu_seqlens_k, "sage_forward_varlen: cu_seqlens is NULL");
-  SAGE_REQUIRE(q8 && qs && k8 && ks && v8t && vs, "sage_forward_varlen: an intermediate pointer is NULL");
-  SAGE_REQUIRE(sage::aligned16(q8) && sage::aligned16(k8) && sage::aligned16(v8t) && sage::aligned16(vs),
-               "sage_forward_varlen: q8 / k8 / v8t / vs must be 16-byte aligned");
-  SAGE_REQUIRE(workspace != nullptr && workspace_bytes >= L.bytes,
-               "sage_forward_varlen: workspace of %lld bytes, the layout needs %lld", (long long)workspace_bytes,
-               (long long)L.bytes);
-  SAGE_REQUIRE(((uintptr_t)workspace & 255u) == 0, "sage_forward_varlen: workspace must be 256-byte aligned");
-  char* ws = static_cast<char*>(workspace);
-  int* hdr = reinterpret_cast<int*>(ws + L.hdr);
-  int* kp = reinterpret_cast<int*>(ws + L.kp);
-  int* order = reinterpret_cast<int*>(ws + L.order);
-  int* tpre = reinterpret_cast<int*>(ws + L.tpre);
-  int* ktab = reinterpret_cast<int*>(ws + L.ktab);
-  int4* tiles = reinterpret_cast<int4*>(ws + L.tiles);
-  hipStream_t st = (hipStream_t)stream;
+  return sage::forward_varlen(q, qss, qsh, k, kss, ksh, v, vss, vsh, out, oss, osh, cu_seqlens_q, cu_seqlens_k, batch, H, Hkv,
+                              total_q, total_k, D, dtype, causal, qs_mul, sage::VarlenRoute{true, 0, 0}, q8, qs, k8, ks, v8t,
+                              vs, workspace, workspace_bytes, stream);
+}
 
-  const int n_kblk = L.tkp / 128;
-  const int64_t n_vs = (int64_t)batch * Hkv * sage::layout_dim(D);
-  const int64_t n_items = std::max<int64_t>(std::max(L.n_blocks, n_kblk), n_vs);
-  const int grid = (int)std::min<int64_t>((n_items + 255) / 256, 4096);
-  if (batch <= sage::VL_WAVE) {
-    hipLaunchKernelGGL(sage::varlen_tables_kernel, dim3(grid), dim3(256), 0, st, cu_seqlens_q, cu_seqlens_k, batch, H,
-                       total_q, total_k, causal ? 1 : 0, hdr, kp, L.n_blocks, n_kblk, tiles, ktab, vs, n_vs);
-  } else {
-    hipLaunchKernelGGL(sage::varlen_meta_kernel, dim3(1), dim3(sage::VL_META_THREADS), 0, st, cu_seqlens_q,
-                       cu_seqlens_k, batch, H, total_q, total_k, hdr, kp, order, tpre);
-    if ((rc = sage::check_launch("varlen meta launch"))) return rc;
-    hipLaunchKernelGGL(sage::varlen_prep_kernel, dim3(grid), dim3(256), 0, st, hdr, cu_seqlens_q, kp, order, tpre, batch,
-                       H, causal ? 1 : 0, L.n_blocks, n_kblk, tiles, ktab, vs, n_vs);
-  }
-  if ((rc = sage::check_launch("varlen table launch"))) return rc;
-  if ((rc = sage::varlen_quant_impl(q, qss, qsh, k, kss, ksh, v, vss, vsh, H, Hkv, total_q, L.tkp, D, dtype, qs_mul,
-                                    cu_seqlens_k, kp, ktab, q8, qs, k8, ks, v8t, vs, stream)))
-    return rc;
-  return sage::attn_varlen_impl(q8, qs, k8, ks, v8t, vs, out, oss, osh, H, Hkv, total_q, L.tkp, D, causal, dtype,
-                                L.n_blocks, tiles, cu_seqlens_q, cu_seqlens_k, kp, stream);
+int sage_forward_varlen_routed(const void* q, int64_t qss, int64_t qsh, const void* k, int64_t kss, int64_t ksh,
+                               const void* v, int64_t vss, int64_t vsh, void* out, int64_t oss, int64_t osh,
+                               const int* cu_seqlens_q, const int* cu_seqlens_k, int batch, int H, int Hkv, int total_q,
+                               int total_k, int D, int dtype, int causal, float qs_mul, int64_t min_kv, int64_t min_work,
+                               int8_t* q8, float* qs, int8_t* k8, float* ks, uint8_t* v8t, float* vs, void* workspace,
+                               int64_t workspace_bytes, void* stream) {
+  sage::clear_error();
+  return sage::forward_varlen(q, qss, qsh, k, kss, ksh, v, vss, vsh, out, oss, osh, cu_seqlens_q, cu_seqlens_k, batch, H, Hkv,
+                              total_q, total_k, D, dtype, causal, qs_mul, sage::VarlenRoute{false, min_kv, min_work}, q8, qs,
+                              k8, ks, v8t, vs, workspace, workspace_bytes, stream);
 }
 
 }  // extern "C"

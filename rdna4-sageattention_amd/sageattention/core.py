@@ -13,7 +13,7 @@ import torch
 from torch.autograd import forward_ad
 
 import cdna4_sage
-from cdna4_sage._attention import row_lse
+from cdna4_sage._attention import packed_pass, row_lse
 
 _LSE_SCORE_BUDGET = 64 * 2**20  # fp32 scores per chunk of the LSE pass (~256 MB)
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
@@ -147,7 +147,7 @@ def sageattn_varlen(
     read back, or with CDNA4_SAGE_VARLEN_ROUTE=0, the packed pass takes every sequence (no host synchronisation; the
     short ones are then quantized too).  Without a gfx950 GPU, or when the longest key sequence is below MIN_KV, every
     sequence goes through sageattn; empty query sequences are skipped."""
-    mk = _int_or_none(max_seqlen_k)
+    mk, seqs = _int_or_none(max_seqlen_k), None
     if q.is_cuda and (mk is None or mk >= cdna4_sage.MIN_KV):
         sync_free = (not cdna4_sage.VARLEN_ROUTE or torch.compiler.is_compiling()
                      or torch.cuda.is_current_stream_capturing())
@@ -155,19 +155,21 @@ def sageattn_varlen(
             if sync_free:
                 return cdna4_sage.attention_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
                                                    sm_scale=sm_scale, is_causal=is_causal)
-            # by the caller's maximum lengths (plain numbers) some sequence may take the kernel: no wait for the offsets
+            # by the caller's maximum lengths (plain numbers) some sequence may take the kernel: no wait for the offsets.
+            # Lengths past the totals are a bound and not a sequence's: what the batch holds is read first then (three
+            # sequences of 900 to 1200 tokens and a maximum of 40960, 8 heads x 64: 224 us, 293 with a pass queued in vain)
             if (cu_seqlens_q.device == q.device and cu_seqlens_k.device == q.device
                     and isinstance(max_seqlen_q, int) and mk is not None
+                    and max_seqlen_q <= q.shape[0] and mk <= k.shape[0]
                     and _kernel_takes(max_seqlen_q, mk, q.shape[1], is_causal)):
-                out = _varlen_overlapped(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, mk, is_causal, sm_scale)
+                out, seqs = _varlen_overlapped(q, k, v, cu_seqlens_q, cu_seqlens_k, is_causal, sm_scale)
                 if out is not None:
                     return out
             else:
                 seqs = _sequences(cu_seqlens_q, cu_seqlens_k)
                 fast = [_kernel_takes(q1 - q0, k1 - k0, q.shape[1], is_causal) for q0, q1, k0, k1 in seqs]
                 if any(fast):
-                    out = cdna4_sage.attention_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
-                                                      sm_scale=sm_scale, is_causal=is_causal)
+                    out = packed_pass(q, k, v, cu_seqlens_q, cu_seqlens_k, sm_scale, is_causal, _route())
                     for (q0, q1, k0, k1), f in zip(seqs, fast):
                         if not f:
                             out[q0:q1] = _one_sequence(q, k, v, q0, q1, k0, k1, is_causal, sm_scale)
@@ -175,7 +177,7 @@ def sageattn_varlen(
         except cdna4_sage.Unsupported:
             pass
     out = torch.empty_like(q)
-    for q0, q1, k0, k1 in _sequences(cu_seqlens_q, cu_seqlens_k):
+    for q0, q1, k0, k1 in seqs or _sequences(cu_seqlens_q, cu_seqlens_k):
         out[q0:q1] = _one_sequence(q, k, v, q0, q1, k0, k1, is_causal, sm_scale)
     return out
 
@@ -187,24 +189,24 @@ def _int_or_none(x):
         return None
 
 
-def _varlen_overlapped(q, k, v, cu_seqlens_q, cu_seqlens_k, max_q, max_k, is_causal, sm_scale):
-    """The routed packed call with the offsets on the GPU: the packed pass is queued before they are read back, and
-    the side stream reads them and runs the sequences that take torch SDPA beside it, so the GPU neither waits for the
-    host nor runs those short, few-workgroup calls alone.  None when the offsets hold no sequence that takes the kernel
-    (the pass's output is then dropped).  Six sequences of 640 (SDPA) to 4608 tokens, 24 heads x 128: 658 -> 575 us per
-    call."""
+def _varlen_overlapped(q, k, v, cu_seqlens_q, cu_seqlens_k, is_causal, sm_scale):
+    """The routed packed call with the offsets on the GPU, and the sequences they hold: the packed pass is queued before
+    they are read back, and the side stream reads them and runs the sequences that take torch SDPA beside it, so the GPU
+    neither waits for the host nor runs those short, few-workgroup calls alone.  Six sequences of 640 (SDPA) to 4608 tokens,
+    24 heads x 128: 658 -> 575 us per call.  The output is None when the offsets hold no sequence that takes the kernel
+    (maximum lengths that are upper bounds); the pass, which follows the same rule, then did nothing, at the price of its
+    five launches (3 us a call among others, 40 alone)."""
     cur, side = torch.cuda.current_stream(q.device), _side_stream(q.device)
     side.wait_stream(cur)  # the inputs, the offsets among them
-    out = cdna4_sage.attention_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_q, max_k, sm_scale=sm_scale,
-                                      is_causal=is_causal)
+    out = packed_pass(q, k, v, cu_seqlens_q, cu_seqlens_k, sm_scale, is_causal, _route())
     with torch.cuda.stream(side):
         seqs = _sequences(cu_seqlens_q, cu_seqlens_k)  # the host waits here: the offsets need no record_stream
         fast = [_kernel_takes(q1 - q0, k1 - k0, q.shape[1], is_causal) for q0, q1, k0, k1 in seqs]
         if not any(fast):
-            return None
+            return None, seqs
         rest = [s for s, f in zip(seqs, fast) if not f]
         if not rest:
-            return out
+            return out, seqs
         for t in (q, k, v):
             t.record_stream(side)
         parts = [_one_sequence(q, k, v, *s, is_causal, sm_scale) for s in rest]
@@ -212,7 +214,12 @@ def _varlen_overlapped(q, k, v, cu_seqlens_q, cu_seqlens_k, max_q, max_k, is_cau
     for (q0, q1, _, _), part in zip(rest, parts):
         out[q0:q1] = part
         part.record_stream(cur)
-    return out
+    return out, seqs
+
+
+def _route():
+    """packed_pass's rule, as _kernel_takes has it."""
+    return cdna4_sage.MIN_KV, cdna4_sage.MIN_WORK
 
 
 def _sequences(cu_seqlens_q, cu_seqlens_k):
