@@ -140,7 +140,10 @@ struct VarlenTiles {
 // layout.  `dout` output channels are written.  c0 = log2(e) / sqrt(head_dim).
 // MASK: a mask (MaskTabs) instead of the causal / padding bound, whose causal flag is folded into its bits: MASK_BOOL
 // (classes 0-2) or MASK_ADD (additive, class 3 as well; apart because its tile body costs the other bodies registers).
-constexpr int MASK_NONE = 0, MASK_BOOL = 1, MASK_ADD = 2;
+// Head dim 256 reads an additive mask whose rows are further apart than a 32-bit offset reaches in a kernel of its own,
+// MASK_ADD_WIDE: with both addresses in one kernel it spills 39 registers instead of 13 (whole calls, against a build with
+// the one: 1.09x and 1.12x slower on the average of dense and of 0 / -inf masks); head dims to 128 hold both.
+constexpr int MASK_NONE = 0, MASK_BOOL = 1, MASK_ADD = 2, MASK_ADD_WIDE = 3;
 constexpr int64_t MASK_ROW_32BIT = 1 << 26;  // 31 rows of at most this many 16-bit elements: a 32-bit byte offset
 // PART: the format of a split tile's partials, fp16 or fp32, or (mask variants) by the argument p32.  Two kernels rather
 // than two epilogues in one: with both, the fp16 launches lost 1.4% (Flux, 158.1 -> 160.4 us; 13.8 -> 14.2 us at
@@ -148,7 +151,7 @@ constexpr int64_t MASK_ROW_32BIT = 1 << 26;  // 31 rows of at most this many 16-
 constexpr int PART_F16 = 0, PART_F32 = 1, PART_ANY = 2, PART_NONE = 3;  // PART_NONE: no split tiles at all
 constexpr int part_format(bool causal, int mask) { return mask ? PART_ANY : causal ? PART_NONE : PART_F16; }
 template <int HD, bool CAUSAL, int OUT_DT, bool VARLEN, int MASK = MASK_NONE, int PART = part_format(CAUSAL, MASK)>
-__global__ __launch_bounds__(ATT_THREADS, (attn_occupancy<layout_dim(HD), MASK == MASK_ADD>())) void attn_kernel(
+__global__ __launch_bounds__(ATT_THREADS, (attn_occupancy<layout_dim(HD), MASK >= MASK_ADD>())) void attn_kernel(
     const int8_t* __restrict__ q8, const float* __restrict__ qs, const int8_t* __restrict__ k8,
     const float* __restrict__ ks, const uint8_t* __restrict__ v8t, const float* __restrict__ vs,
     uint16_t* __restrict__ out, int64_t osb, int64_t oss, int64_t osh, float* __restrict__ lse, int H, int Hkv,
@@ -379,7 +382,7 @@ __global__ __launch_bounds__(ATT_THREADS, (attn_occupancy<layout_dim(HD), MASK =
       o_ = (uint32_t)(((min(q0 + (ql_ & 31), Sq - 1) - qw_) * (int)mt.psq + 8 * (ql_ >> 5)) * 2);          \
     }                                                                                                      \
     asm volatile("" : "+s"(p_), "+v"(o_));                                                                 \
-    if (mt.vsq > MASK_ROW_32BIT && !part_) {                                                               \
+    if ((D <= 128 || MASK == MASK_ADD_WIDE) && mt.vsq > MASK_ROW_32BIT && !part_) {                        \
       const int ql_ = lane_id(), qw_ = min(q0, Sq - 1);                                                    \
       const uint8_t* r_ = p_ + ((min(q0 + (ql_ & 31), Sq - 1) - qw_) * mt.vsq + 8 * (ql_ >> 5)) * 2;       \
       _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) (BW)[i_] = load16_2aligned(r_ + 32 * i_);           \
@@ -713,7 +716,7 @@ __global__ __launch_bounds__(ATT_THREADS, (attn_occupancy<layout_dim(HD), MASK =
     } else if (cs == 2) {
       const uint32_t mw = load_global_u32(mbase + (moff + 8u * (uint32_t)ts));
       SAGE_TILE_PASSES(ts, 2, mw, bw_none, wide);
-    } else if (MASK == MASK_ADD && cs == 3) {
+    } else if (MASK >= MASK_ADD && cs == 3) {
       v4i bias_w[4];
       SAGE_LOAD_BIAS(ts, bias_w);
       SAGE_TILE_PASSES(ts, 3, 0u, bias_w, wide);
@@ -831,7 +834,7 @@ __global__ __launch_bounds__(ATT_THREADS, (attn_occupancy<layout_dim(HD), MASK =
       // a run of class 3 (additive mask): the lane's 64 bytes of bias values of the tile are loaded before the next
       // tile's direct loads, which are always issued here (the last iteration reloads its own tile into the idle
       // buffer), so the wait for the values counts the direct loads behind them and does not wait for them
-      for (; MASK == MASK_ADD && t < t_hi && c_nxt == 3; ++t) {
+      for (; MASK >= MASK_ADD && t < t_hi && c_nxt == 3; ++t) {
         v4i bias_w[4];
         SAGE_LOAD_BIAS(t, bias_w);
         const int tn_ = min(t + 1, t_hi - 1);
@@ -1328,9 +1331,11 @@ static int launch_attn_mask(const int8_t* q8, const float* qs, const int8_t* k8,
   const float c0 = logit_scale_base(hd);
   uint16_t* o = static_cast<uint16_t*>(out);
   float* part = static_cast<float*>(workspace);
-  hipLaunchKernelGGL((attn_kernel<HD, false, OUT_DT, false, ADDITIVE ? MASK_ADD : MASK_BOOL>), dim3(blocks),
-                     dim3(ATT_THREADS), 0, st, q8, qs, k8, ks, v8t, vs, o, osb, oss, osh, nullptr, H, Hkv, Sq, Skv,
-                     kv_pad(Skv), q_tiles, p.n_tiles, p.n_full, p.chunks, (int)p.p32, part, c0, hd, VarlenTiles{}, mt,
+  auto* kernel = attn_kernel<HD, false, OUT_DT, false, ADDITIVE ? MASK_ADD : MASK_BOOL>;
+  if constexpr (ADDITIVE && HD == 256)
+    if (mt.vsq > MASK_ROW_32BIT) kernel = attn_kernel<HD, false, OUT_DT, false, MASK_ADD_WIDE>;
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(ATT_THREADS), 0, st, q8, qs, k8, ks, v8t, vs, o, osb, oss, osh, nullptr, H,
+                     Hkv, Sq, Skv, kv_pad(Skv), q_tiles, p.n_tiles, p.n_full, p.chunks, (int)p.p32, part, c0, hd, VarlenTiles{}, mt,
                      mt.bits, mt.cls, mt.range);
   if (n_split > 0) {
     if ((rc = check_launch("masked attention launch"))) return rc;

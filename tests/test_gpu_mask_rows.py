@@ -57,8 +57,9 @@ def test_mask_layouts_give_the_same_bits(dev, B, H, Sq, Skv, D, dt, causal, rows
     assert torch.equal(cdna4_sage.attention(q, k, v, "HND", is_causal=causal, attn_mask=full.contiguous()), out)
 
 
-def test_mask_rows_further_apart_than_32_bits(dev):
-    B, H, Sq, Skv, D = 1, 2, 40, 200, 64
+@pytest.mark.parametrize("D", [64, 256])
+def test_mask_rows_further_apart_than_32_bits(dev, D):
+    B, H, Sq, Skv = 1, 2, 40, 200
     (q, k, v), g = _qkv(dev, B, H, Sq, Skv, D, BF16, 3)
     mask = _values(g, (Sq, Skv), dev, BF16)
     out = cdna4_sage.attention(q, k, v, "HND", attn_mask=mask)
