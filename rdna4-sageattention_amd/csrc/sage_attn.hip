@@ -140,6 +140,9 @@ struct VarlenTiles {
 // layout.  `dout` output channels are written.  c0 = log2(e) / sqrt(head_dim).
 // MASK: a mask (MaskTabs) instead of the causal / padding bound, whose causal flag is folded into its bits: MASK_BOOL
 // (classes 0-2) or MASK_ADD (additive, class 3 as well; apart because its tile body costs the other bodies registers).
+// At head dim 96 the compiler schedules the two bodies of MASK_BOOL worse than the three of MASK_ADD, and bool masks run on
+// that one as well (padding, 12 heads x 4167: whole call 69 us on the former, 64 on the latter; 380 to 512 tiles, 1.03x on
+// the average of 240 random calls).
 // Head dim 256 reads an additive mask whose rows are further apart than a 32-bit offset reaches in a kernel of its own,
 // MASK_ADD_WIDE: with both addresses in one kernel it spills 39 registers instead of 13 (whole calls, against a build with
 // the one: 1.09x and 1.12x slower on the average of dense and of 0 / -inf masks); head dims to 128 hold both.
@@ -1331,7 +1334,7 @@ static int launch_attn_mask(const int8_t* q8, const float* qs, const int8_t* k8,
   const float c0 = logit_scale_base(hd);
   uint16_t* o = static_cast<uint16_t*>(out);
   float* part = static_cast<float*>(workspace);
-  auto* kernel = attn_kernel<HD, false, OUT_DT, false, ADDITIVE ? MASK_ADD : MASK_BOOL>;
+  auto* kernel = attn_kernel<HD, false, OUT_DT, false, ADDITIVE || HD == 96 ? MASK_ADD : MASK_BOOL>;
   if constexpr (ADDITIVE && HD == 256)
     if (mt.vsq > MASK_ROW_32BIT) kernel = attn_kernel<HD, false, OUT_DT, false, MASK_ADD_WIDE>;
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(ATT_THREADS), 0, st, q8, qs, k8, ks, v8t, vs, o, osb, oss, osh, nullptr, H,
