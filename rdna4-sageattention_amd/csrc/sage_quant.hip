@@ -431,16 +431,16 @@ constexpr int V_SLICE = 16;  // channels per workgroup
 // V_SHORT_BYTES, since a slice's 32-byte row pieces use a quarter of each line they touch.  Whole call, two launches
 // against one (one MI355X, bf16): 1x8x1024x64 20.7 -> 19.6 us, 2x20x1024x64 (5 MB of V) 33.7 -> 30.8, 1x24x1024x128
 // (6 MB) 41.7 -> 39.7, 2x10x4096 queries x 77 keys x 64 22.3 -> 18.9, 1x12x8192 x 256 keys x 256 63.1 -> 58.1; past the
-// line 2x40x640x128 (13 MB) 40.8 -> 41.7, 2x40x1024x128 (21 MB) 62.4 -> 64.8.  A quarter of head dim 96's slices are padding:
-// 3/4 of the rows (24 heads x 512 queries x 1024 keys 30.7 -> 30.0; 40 x 512 x 640 32.7 -> 33.9, 40 x 512 x 1024 37.5 -> 39.1).
-// Slices past V_SHORT_SLICES queue up: of 256 channels (16 slices a head), 64 queries x 77 keys, 40 heads 23.8 -> 21.7 us, 64
-// heads 24.7 -> 25.4, 160 heads 30.8 -> 38.2; of 128, 80 heads 17.7 -> 16.6, 160 heads 20.6 -> 21.5.
+// line 2x40x640x128 (13 MB) 40.8 -> 41.7, 2x40x1024x128 (21 MB) 62.4 -> 64.8.
+// Slices past V_SHORT_SLICES (three a CU) queue up: of 256 channels (16 slices a head), 64 queries x 77 keys, 40 heads 23.8
+// -> 21.7 us, 48 heads (83 x 19) 23.4 -> 22.0, 64 heads 24.7 -> 25.4, 160 heads 30.8 -> 38.2; of 128, 80 heads 17.7 -> 16.6,
+// 160 heads 20.6 -> 21.5.
 constexpr int64_t V_SHORT_BYTES = 8ll << 20;
-constexpr int64_t V_SHORT_SLICES = 640;
+constexpr int64_t V_SHORT_SLICES = 768;
 static inline bool v_short(int B, int Hkv, int Skv, int D) {
   const int64_t heads = (int64_t)B * Hkv;
   return Skv <= V_SHORT_KEYS && heads * (layout_dim(D) / V_SLICE) <= V_SHORT_SLICES &&
-         heads * Skv * layout_dim(D) * 2 <= (D == 96 ? V_SHORT_BYTES / 4 * 3 : V_SHORT_BYTES);
+         heads * Skv * D * 2 <= V_SHORT_BYTES;
 }
 
 template <int D, int DT>

@@ -15,9 +15,8 @@ CASES = [(1, 2, 2, 70, n, D, dt, layout) for n, D, dt, layout in (
 CASES += [(2, 6, 3, 300, 333, 128, "bf16", "NHD"),
           (2, 16, 16, 64, 1024, 128, "bf16", "HND"),    # 8 MiB of V: the last one-launch size
           (1, 33, 33, 64, 1024, 128, "bf16", "HND"),    # past it
-          (1, 24, 24, 64, 1024, 96, "bf16", "HND"), (1, 25, 25, 64, 1024, 96, "bf16", "HND"),   # the same at head dim 96
-          (1, 40, 40, 64, 77, 256, "f16", "HND"), (1, 41, 41, 64, 77, 256, "f16", "NHD"),       # 640 slices, and past it
-          (2, 80, 40, 64, 77, 128, "bf16", "NHD"), (3, 54, 54, 64, 77, 64, "bf16", "HND")]
+          (2, 24, 24, 64, 77, 256, "f16", "HND"), (1, 49, 49, 64, 77, 256, "f16", "NHD"),   # 768 slices, and past it
+          (3, 64, 32, 64, 77, 96, "bf16", "NHD"), (3, 65, 65, 64, 77, 64, "bf16", "HND")]
 
 
 @pytest.mark.parametrize("B,H,Hkv,Sq,Skv,D,dt,layout", CASES)
