@@ -1057,13 +1057,21 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict
 //     / 124), or 32 inside the first round (d64, L 64, n 640: 73 / 86; d128, n 640: L 20 47 / 44) and at two workgroups
 //     per CU unless c is a short last round or at most cus / 8 (d256, n 896: L 20 111 / 103, L 32 152 / 149, L 40 183 /
 //     185; n 784, c = 16: L 20 94 / 99).
-//  4. Two ranges of the last round from L 128 where the round leaves CUs without a tile, r <= cus, or without the second,
-//     0 < c <= 3/4 cus; fp16 partials.  d256, n 768: L 80 299 / 295, L 96 350 / 360 (whole calls: L 96 391 / 388, L 192
-//     716 / 736); d64, n 448, L 128 136 / 138; d64, n 1440, L 256 662 / 672.  d64, n 1536 (c = 0), L 512 1307 / 1275.
+//  4. Ranges of the last round, fp16 partials, from L 96 where it leaves CUs without a tile, r < cus (d256, n 688: L 80 278 /
+//     284, L 96 327 / 339; n 720, L 119, whole call 488 / 509), from L 128 where it leaves them without a second, r = cus or
+//     0 < c <= 3/4 cus (d256, n 768, whole calls: L 96 391 / 388, L 192 716 / 736; d64, n 448, L 128 136 / 138; d64, n
+//     1440, L 256 662 / 672).  d64, n 1536 (c = 0), L 512 1307 / 1275.
 //  5. Causal: every tile of launches of at most cus tiles, the longer the key range the more tiles (L >= n / 4 at 256
 //     CUs), fp32 partials.  d128, 192 tiles of a 700-row chunk against 8192 keys (4 ranges): 80 / 120; square 8 x 2048
 //     (128 tiles, L 32): 31 / 35; below the line 16 x 2048 (256 tiles, L 32): 41 / 36; past one tile per CU, 384 tiles of
-//     1500 rows against 9001 keys (2 ranges): 152 / 149, and square 8 x 8192 (512 tiles): 138 / 126.
+//     1500 rows against 9001 keys (2 ranges): 152 / 149, and square 8 x 8192 (512 tiles): 138 / 126.  Two ranges at two
+//     workgroups per CU past 7/8 cus, of chunks (tiles of like length), from L >= 5/16 n (whole calls, d256, 64 heads to 8,
+//     n 256: L 67 148 / 141; square 8 x 4034: 109 / 113).
+//     Over slots / n ranges; over one unit a CU, whose merge is shorter, for at most 5/16 cus tiles below L 48, and at two
+//     workgroups per CU for cus / 2 below L 40 (d256, square 4 x 2976, n 96, L 47: 66 against 61 by slots / n).  Whole calls
+//     by one unit a CU, by slots / n ranges and whole: 32 heads to 4, d128, n 64, L 28 33.4, 35.7, 40.7; d256, n 128, L 32
+//     64.7, 72.3, 69.3; 8 heads, d128, n 112, L 28 39.5, 37.0, 42.4.
+//     Past cus / 12 tiles from L 10 (d128, n 32: L 8 20.0 / 19.4, L 10 21.6 / 22.2).
 // Masked launches plan with the causal flag folded into the mask, rules 1 to 4, less what shorter walks make dearer: rule
 // 2's three ranges below 2 cus from L 48 (d64, n 320, L 40 with 5/8 of the keys, whole call 47 / 42), its units one a CU
 // only where neither the causal flag nor a bool mask's rows shorten some walks (d256, n 576, L 18, causal: 107 / 99), and no
@@ -1126,9 +1134,11 @@ static int make_plan(int B, int H, int Sq, int Skv, AttnPlan* p, int walks = WAL
   const int most = min(kv_tiles / 4, ATT_MAX_CHUNKS);
   int rem = 0, chunks = 1;
   if (CAUSAL) {
-    if (n <= cus && (int64_t)kv_tiles * cus >= 64 * (int64_t)n) {  // rule 5
+    const int slope = per_cu <= 2 && 8 * n > 7 * cus && 2 * (int64_t)Sq <= Skv ? 80 : 64;
+    if (n <= cus && kv_tiles >= (12 * n <= cus ? 8 : 10) && (int64_t)kv_tiles * cus >= slope * (int64_t)n) {  // rule 5
+      const bool one_each = 16 * n <= 5 * cus ? kv_tiles < 48 : per_cu <= 2 && 2 * n <= cus && kv_tiles < 40;
       rem = n;
-      chunks = min(slots / n, most);
+      chunks = min((one_each ? cus : slots) / n, most);
       p->p32 = true;
     }
   } else if (n <= cus) {  // rule 1
@@ -1148,7 +1158,7 @@ static int make_plan(int B, int H, int Sq, int Skv, AttnPlan* p, int walks = WAL
       past = 2 * c <= cus && L >= (n < slots || (per_cu <= 2 && c != r && 8 * c > cus) ? 32 : 20);
     }
     past = past && c > 0 && walks != WALKS_DIFFER;
-    const bool two = ranges >= 2 && L >= 128 && (r <= cus || (c > 0 && 4 * c <= 3 * cus));
+    const bool two = ranges >= 2 && L >= (r < cus ? 96 : 128) && (r <= cus || (c > 0 && 4 * c <= 3 * cus));
     if (round || (two && !past)) {  // rules 2 and 4
       rem = r;
       chunks = min(ranges, most);

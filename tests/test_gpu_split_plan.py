@@ -159,9 +159,25 @@ def test_three_ranges_of_head_dim_256_against_whole_tiles(dev):
     (1, 16, 4352, 16, 256, 512, 4, False), (1, 16, 4352, 20, 256, 512, 5, False),
     (1, 16, 7168, 31, 256, 896, 1, False), (1, 16, 7168, 32, 256, 768, 2, True),   # two workgroups per CU
     (1, 16, 6272, 20, 256, 768, 5, True),
+    (1, 12, 7680, 95, 256, 720, 1, False), (1, 12, 7680, 96, 256, 512, 2, False),  # 208 tiles: CUs without one
 ])
 def test_plan_of_short_walks(dev, B, H, Sq, L, D, n_full, chunks, fp32):
     full, ch, ws = _capi.attn_plan(dev.index or 0, B, H, Sq, L * 64, D, 0)
     assert (full, ch) == (n_full, chunks)
     rem, dl = B * H * ((Sq + 127) // 128) - full, _capi.layout_dim(D)
     assert ws == (rem * ch * 128 * ((4 if fp32 else 2) * dl + 8) if ch > 1 else 0)
+
+
+@pytest.mark.parametrize("H,Sq,L,D,chunks", [
+    (8, 250, 7, 64, 1), (8, 250, 8, 64, 2), (8, 500, 9, 128, 1), (8, 500, 10, 128, 2),           # 16 and 32 tiles
+    (32, 250, 15, 256, 1), (32, 250, 16, 256, 4), (8, 1250, 47, 128, 3), (8, 1250, 48, 128, 9),  # 64 and 80
+    (32, 350, 23, 128, 1), (32, 350, 24, 128, 6), (32, 500, 31, 256, 1), (32, 500, 32, 256, 2),  # 96 and 128
+    (32, 500, 39, 256, 2), (32, 500, 40, 256, 4), (32, 1000, 63, 128, 1), (32, 1000, 64, 128, 3),
+    (32, 1000, 79, 256, 1), (32, 1000, 80, 256, 2), (32, 850, 55, 256, 1), (32, 850, 56, 256, 2),  # 256 and 224
+    (8, 4096, 64, 256, 2),
+])
+def test_causal_plan_of_short_walks(dev, H, Sq, L, D, chunks):
+    n = H * ((Sq + 127) // 128)
+    full, ch, ws = _capi.attn_plan(dev.index or 0, 1, H, Sq, L * 64, D, True)
+    assert (full, ch) == (n if chunks == 1 else 0, chunks)
+    assert ws == (n * ch * 128 * (4 * _capi.layout_dim(D) + 8) if ch > 1 else 0)
