@@ -202,6 +202,21 @@ def test_varlen_validates_before_launching():
     assert call(total_q=0) == _capi.SAGE_ERR_INVALID
 
 
+def test_routed_varlen_validates_before_launching():
+    """sage_forward_varlen_routed refuses what sage_forward_varlen refuses, whatever its route."""
+    lib = _capi.lib()
+    _, ws_bytes = _capi.varlen_layout(2, 4, 2, 256, 256)
+    args = dict(q=P, qss=512, qsh=128, k=P, kss=256, ksh=128, v=P, vss=256, vsh=128, out=P, oss=512, osh=128,
+                cu_q=P, cu_k=P, batch=2, H=4, Hkv=2, total_q=256, total_k=256, D=128, dtype=0, causal=1, qs_mul=1.0,
+                min_kv=1024, min_work=1 << 26, q8=P, qs=P, k8=P, ks=P, v8t=P, vs=P, ws=P, ws_bytes=ws_bytes, stream=None)
+    for kw, code, text in (({"D": 80}, _capi.SAGE_ERR_UNSUPPORTED, "head_dim 80"),
+                           ({"q": P + 8}, _capi.SAGE_ERR_INVALID, "16-byte"),
+                           ({"cu_q": None}, _capi.SAGE_ERR_INVALID, "cu_seqlens"),
+                           ({"ws_bytes": ws_bytes - 1, "min_kv": -1}, _capi.SAGE_ERR_INVALID, "workspace"),
+                           ({"qs_mul": 0.0, "min_work": 1 << 62}, _capi.SAGE_ERR_INVALID, "qs_mul")):
+        assert lib.sage_forward_varlen_routed(*dict(args, **kw).values()) == code and text in _err()
+
+
 def test_masked_forward_validates_before_launching():
     """sage_forward_masked / sage_mask_workspace reject bad shapes, strides and pointers with a code and a message
     before the first HIP call (on this GPU-less machine any later step would fail with a HIP error instead)."""
