@@ -599,7 +599,7 @@ __global__ __launch_bounds__(ATT_THREADS, (attn_occupancy<layout_dim(HD), MASK >
     /* p = exp2(arg); each block's fp32 sum starts from its first p (0 + p is p).  Up to head dim 128 and   \
        without a mask all 32 exponent arguments are formed before the first exponential (SAGE_PHASE_FENCE):  \
        interleaved, each v_exp_f32 waits on the FMA just before it, which three waves per SIMD do not hide.   \
-       The mask variant (three tile bodies) and head dim 256 hold more registers and would spill with it. */ \
+       The mask variants (two or three tile bodies) and head dim 256 hold more registers and would spill.   */ \
     /* a wide wave reads F - c after the block maxima (which order the seeded patterns as ints) and drops the \
        seed term: the offsets are then -(cl * m) after this pass's update, -inf for a slow pass's block 1 */ \
     if ((MODE) != 3 && (WIDE)) {                                                                           \

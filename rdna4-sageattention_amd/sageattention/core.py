@@ -195,7 +195,7 @@ def _varlen_overlapped(q, k, v, cu_seqlens_q, cu_seqlens_k, is_causal, sm_scale)
     neither waits for the host nor runs those short, few-workgroup calls alone.  Six sequences of 640 (SDPA) to 4608 tokens,
     24 heads x 128: 658 -> 575 us per call.  The output is None when the offsets hold no sequence that takes the kernel
     (maximum lengths that are upper bounds); the pass, which follows the same rule, then did nothing, at the price of its
-    five launches (3 us a call among others, 40 alone)."""
+    launches (3 us a call among others, 40 alone)."""
     cur, side = torch.cuda.current_stream(q.device), _side_stream(q.device)
     side.wait_stream(cur)  # the inputs, the offsets among them
     out = packed_pass(q, k, v, cu_seqlens_q, cu_seqlens_k, sm_scale, is_causal, _route())
